@@ -6,28 +6,22 @@
 // Data layout in HBM (one block, haloed extents X = nx+2, Y = ny+2, Z = nz+2, m = X*Y*Z):
 //   natural: the reference's arrays, x fastest: Val(m, 7) column-major for JacTMom and
 //     JacTPot, Val(m, 2) for JacFall; vectors ncomp x m; LU factors ncomp*ncomp x ncell.
-//   skewed (Gauss-Seidel only): row iy, step s = ix + iz, level iz:
-//     k = (iy*S + s)*Z + iz, S = X + Z - 1.  A wavefront owns one y-row, its 64 lanes the
-//     z-levels (iz = lane + 64*slot); at step s every lane updates cell (s - iz, iy, iz),
-//     so one step is one contiguous run of Z entries.  The coefficients are stored per
-//     row of the matrix (w_d[k] = A(r, r + DiagPtr(d))), so a step reads 7 contiguous
-//     runs.  The skew costs (Y*S*Z)/m ~ 1 + Z/X of padding.
+//   skewed (Gauss-Seidel only): level k, y-tile jt of TW columns j, row h = i + jj of
+//     the tile (jj the column within it), 64 entries per row: the cells of one step of a
+//     wavefront whose lanes are the columns (lane l at cell i = step - l) are one contiguous
+//     run.  A matrix holds kCoefWords such runs per row, one after the other.  The skew costs
+//     1 + (TW-1)/X of padding; a step reads whole 128-byte lines.
 //
-// The Gauss-Seidel sweep is the reference's lexicographic forward sweep.  Cell (ix,iy,iz)
-// needs the new values of (ix-1), (iy-1), (iz-1) and the old ones of (ix+1), (iy+1),
-// (iz+1), so every cell of the hyperplane ix+iy+iz = h can be updated at once.  A sweep is
-// t = b - U x_old (a parallel pass) followed by the forward substitution, pipelined over
-// rows: the wavefront of row iy runs one step behind the one of row iy-1.  Inside a
-// workgroup the new values of row iy-1 arrive through LDS (one barrier per step); between
-// workgroups through a boundary-row buffer whose entries carry their own readiness (a
-// sentinel until written).  Workgroups take their row block from an atomic ticket, so a
-// workgroup only ever waits for one that started before it.  Every wait is bounded: past
-// the limit the kernel records an error and stops waiting, so every wave reaches the end.
+// The Gauss-Seidel sweep is the reference's lexicographic forward sweep.  Cell (i, j, k)
+// needs the new values of (i-1), (j-1), (k-1) and the old ones of (i+1), (j+1), (k+1), so
+// every cell of the hyperplane i+j+k = h can be updated at once, and the next sweep can
+// follow two hyperplanes behind: see k_gs_tiles.
 //
 // Products and sums are not contracted (no FMA) in the operator, the sweep and the
 // vector updates, so they round as the reference's separate multiplies and adds.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -50,8 +44,16 @@ struct Ops {
 };
 
 struct Dims {
-  int nx, ny, nz, X, Y, Z, S;
-  long m, ncell, sks;  // sks = Y*S*Z
+  int nx, ny, nz, X, Y, Z;
+  int TW, NJ, HL;         // skewed layout: columns per y-tile, y-tiles, rows per tile and level
+  long m, ncell, slots;   // slots = Z*NJ*HL*64
+};
+
+// Components that go through the sweeps together, one or two per group: two share a matrix
+// (the same operator); a component left over fills both places of its group.
+struct Groups {
+  int n;
+  int c[kMaxComp][2];
 };
 
 __device__ __forceinline__ bool is_interior(const Dims& d, long r, int& i, int& j, int& k) {
@@ -125,50 +127,156 @@ __global__ __launch_bounds__(256) void k_matvec(Dims d, const double* __restrict
   for (int c = 0; c < NC; ++c) y[c * d.m + r] = x[c * d.m + r] + s[c];
 }
 
-// ------------------------------------------------------------------ skewed layout
-__device__ __forceinline__ long skew_of(const Dims& d, long r) {
-  const int i = (int)(r % d.X);
-  const long t = r / d.X;
-  const int j = (int)(t % d.Y), k = (int)(t / d.Y);
-  return ((long)j * d.S + (i + k)) * d.Z + k;
+// ------------------------------------------------------------------ division
+// t / dg from y = 1/dg (correctly rounded): two residual corrections of t*y.  The first leaves
+// a quotient within an ulp and the second rounds correctly (Markstein, IBM J. Res. Dev. 34,
+// 1990), as long as no residual underflows: |t| above 2^-960 and |dg| within 2^+-500 (the
+// set-up notes a matrix with another diagonal, and the sweeps then divide).  Five dependent
+// operations in the sweep's serial chain instead of the division's dozen.  The caller divides
+// where the result is NaN, infinite or subnormal (gs_odd).  The sign is that of t*y, also for
+// a zero.
+__device__ __forceinline__ double gs_divide(double t, double dg, double y) {
+  const double q0 = t * y;
+  const double q1 = __builtin_fma(__builtin_fma(-q0, dg, t), y, q0);
+  const double q2 = __builtin_fma(__builtin_fma(-q1, dg, t), y, q1);
+  return __builtin_copysign(q2, q0);
+}
+__device__ __forceinline__ bool gs_odd(double q) {
+  return __builtin_amdgcn_class(q, 0x003 | 0x204 | 0x090);  // NaN, infinite, subnormal
+}
+__device__ __forceinline__ bool gs_plain_diag(double dg) {
+  const double m = fabs(dg);
+  return m >= 0x1p-500 && m <= 0x1p500;
 }
 
-// Row coefficients w_q[k] = A(r, r + DiagPtr(q)) = Val(r + DiagPtr(q), q) of every
-// valid skewed slot (padding slots stay 0).
-__global__ void k_skew_coef(Dims d, const double* __restrict__ val, double* __restrict__ w) {
-  const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= d.m) return;
-  const long XY = (long)d.X * d.Y;
-  const long off[7] = {-XY, -(long)d.X, -1, 0, 1, (long)d.X, XY};
-  const long k = skew_of(d, r);
+// ------------------------------------------------------------------ skewed layout
+// Slot of cell (i, j, k) within an array of one word per cell: y-tile jt = j / TW, column
+// jj = j - jt*TW, row h = i + jj of the tile's HL = X + TW - 1 rows.
+constexpr int kRow = 64;       // entries of a row of the skewed layout
+constexpr int kCoefWords = 8;  // words per cell of a skewed matrix: see k_skew_coef
+
+// Place of word q of a cell within a matrix row: the words lie in pairs, so that a lane takes
+// two with one 16-byte load (a wavefront's load costs the address unit the same 16 cycles
+// whatever its width).
+__device__ __forceinline__ constexpr int coef_word(int q) { return (q >> 1) * (2 * kRow) + (q & 1); }
+
+__device__ __forceinline__ long slot_row(const Dims& d, int jt, int h, int k) {
+  return ((long)k * d.NJ + jt) * d.HL + h;
+}
+
+// Natural rows j of one (level, y-tile) to skewed rows h, 64 rows h at a time: the loads run
+// along x, the stores along y, transposed through LDS (a thread per cell would scatter one
+// of the two).  get(jj, i) gives the value of cell (i, j0 + jj); put(h, jj, v) stores it.
+// Slots outside the block (i out of range) are not written and never used.
+constexpr int kTileH = 64;
+__host__ __device__ inline int h_blocks(const Dims& d) { return (d.HL + kTileH - 1) / kTileH; }
+template <typename Get, typename Put>
+__device__ __forceinline__ void skew_tile(const Dims& d, int jt, int h0, double (*t)[kTileH + 1],
+                                          Get&& get, Put&& put) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int rows = min(d.TW, d.Y - jt * d.TW);
+  for (int jj = wv; jj < rows; jj += 4) {
+    const int i = h0 + lane - jj;
+    if (i >= 0 && i < d.X) t[jj][lane] = get(jj, i);
+  }
+  __syncthreads();
+  for (int hh = wv; hh < kTileH; hh += 4) {
+    const int h = h0 + hh, i = h - lane;
+    if (lane < rows && h < d.HL && i >= 0 && i < d.X) put(h, lane, t[lane][hh]);
+  }
+  __syncthreads();
+}
+
+// Row coefficients A(r, r + DiagPtr(q)) = Val(r + DiagPtr(q), q) of every cell, in the order
+// the sweep uses them: +1, +X, +XY, -XY, -X, -1, diagonal, and the diagonal's reciprocal.  A coupling that leaves the block is +0 (the set-up has checked that it is
+// zero; its sign must not reach the sweep's sums).  Grid (y-tiles x runs of 64 h, 1, levels).
+// *odd is set where a diagonal is too large or too small for gs_divide.
+__global__ __launch_bounds__(256) void k_skew_coef(Dims d, const double* __restrict__ val,
+                                                   double* __restrict__ w, int* odd) {
+  __shared__ double t[64][kTileH + 1];
+  const int nh = h_blocks(d), jt = blockIdx.x / nh, h0 = (blockIdx.x - jt * nh) * kTileH;
+  const int k = blockIdx.z;
+  const int di[7] = {1, 0, 0, 0, 0, -1, 0}, dj[7] = {0, 1, 0, 0, -1, 0, 0},
+            dk[7] = {0, 0, 1, -1, 0, 0, 0}, dq[7] = {4, 5, 6, 0, 1, 2, 3};
 #pragma unroll
   for (int q = 0; q < 7; ++q) {
-    const long src = r + off[q];
-    w[q * d.sks + k] = (src >= 0 && src < d.m) ? val[q * d.m + src] : 0.0;
+    skew_tile(
+        d, jt, h0, t,
+        [&](int jj, int i) {
+          const int i2 = i + di[q], j2 = jt * d.TW + jj + dj[q], k2 = k + dk[q];
+          const bool in = i2 >= 0 && i2 < d.X && j2 >= 0 && j2 < d.Y && k2 >= 0 && k2 < d.Z;
+          return in ? val[(long)dq[q] * d.m + i2 + (long)d.X * (j2 + (long)d.Y * k2)] : 0.0;
+        },
+        [&](int h, int jj, double v) {
+          double* row = w + slot_row(d, jt, h, k) * (kCoefWords * kRow) + 2 * jj;
+          row[coef_word(q)] = v;
+          if (q == 6) {
+            row[coef_word(7)] = 1.0 / v;
+            if (!gs_plain_diag(v)) *odd = 1;
+          }
+        });
   }
 }
-// JacFall rows: f0 = its diagonal at r, f1 = its coupling of row r to r + XY.
-__global__ void k_skew_fall(Dims d, const double* __restrict__ fall, double* __restrict__ wf) {
-  const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= d.m) return;
-  const long XY = (long)d.X * d.Y;
-  const long k = skew_of(d, r);
-  wf[k] = fall[r];
-  wf[d.sks + k] = (r + XY < d.m) ? fall[d.m + r + XY] : 0.0;
+// JacFall rows: word 0 its diagonal, word 1 its coupling of row r to r + XY.
+__global__ __launch_bounds__(256) void k_skew_fall(Dims d, const double* __restrict__ fall,
+                                                   double* __restrict__ wf) {
+  __shared__ double t[64][kTileH + 1];
+  const int nh = h_blocks(d), jt = blockIdx.x / nh, h0 = (blockIdx.x - jt * nh) * kTileH;
+  const int k = blockIdx.z;
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+    skew_tile(
+        d, jt, h0, t,
+        [&](int jj, int i) {
+          const int k2 = k + q;
+          return k2 < d.Z ? fall[q * d.m + i + (long)d.X * (jt * d.TW + jj + (long)d.Y * k2)] : 0.0;
+        },
+        [&](int h, int jj, double v) {
+          wf[slot_row(d, jt, h, k) * (2 * kRow) + 2 * jj + q] = v;
+        });
 }
-__global__ void k_skew_vec(Dims d, int nc, const double* __restrict__ v, double* __restrict__ vs) {
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (long)nc * d.m) return;
-  const long c = e / d.m, r = e - c * d.m;
-  vs[c * d.sks + skew_of(d, r)] = v[e];
+// Grid z: levels x groups x NC.
+template <int NC>
+__global__ __launch_bounds__(256) void k_skew_vec(Dims d, Groups gr, const double* __restrict__ v,
+                                                  double* __restrict__ vs) {
+  __shared__ double t[64][kTileH + 1];
+  const int nh = h_blocks(d), jt = blockIdx.x / nh, h0 = (blockIdx.x - jt * nh) * kTileH;
+  const int e = blockIdx.z / d.Z, k = blockIdx.z - e * d.Z, g = e / NC, h = e - g * NC;
+  const double* const src = v + (long)gr.c[g][h] * d.m;
+  double* const dst = vs + g * d.slots * NC + h;
+  skew_tile(
+      d, jt, h0, t,
+      [&](int jj, int i) { return src[i + (long)d.X * (jt * d.TW + jj + (long)d.Y * k)]; },
+      [&](int h, int jj, double x) { dst[(slot_row(d, jt, h, k) * kRow + jj) * NC] = x; });
 }
-// Back to the natural layout with the six halo faces zero (PSolveSp :734-739).
-__global__ void k_unskew(Dims d, int nc, const double* __restrict__ vs, double* __restrict__ v) {
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (long)nc * d.m) return;
-  const long c = e / d.m, r = e - c * d.m;
-  int i, j, k;
-  v[e] = is_interior(d, r, i, j, k) ? vs[c * d.sks + skew_of(d, r)] : 0.0;
+// Back to the natural layout with the six halo faces zero (PSolveSp :734-739).  Grid
+// (y-tiles x runs of 64 cells along x, 1, levels x groups x NC).
+template <int NC>
+__global__ __launch_bounds__(256) void k_unskew(Dims d, Groups gr, const double* __restrict__ vs,
+                                                double* __restrict__ v) {
+  __shared__ double t[2 * kTileH][64 + 1];
+  const int nx = (d.X + kTileH - 1) / kTileH, jt = blockIdx.x / nx;
+  const int i0 = (blockIdx.x - jt * nx) * kTileH;
+  const int e = blockIdx.z / d.Z, k = blockIdx.z - e * d.Z, g = e / NC, n = e - g * NC;
+  const int c = gr.c[g][n];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  const int rows = min(d.TW, d.Y - jt * d.TW);
+  const double* src = vs + g * d.slots * NC + n;
+  const bool inner_k = k >= 1 && k <= d.nz;
+  if (inner_k)
+    for (int hh = wv; hh < kTileH + d.TW - 1; hh += 4) {
+      const int h = i0 + hh, i = h - lane;
+      if (lane < rows && h < d.HL && i >= i0 && i < d.X)
+        t[hh][lane] = src[(slot_row(d, jt, h, k) * kRow + lane) * NC];
+    }
+  __syncthreads();
+  const int i = i0 + lane;
+  if (i >= d.X) return;
+  for (int jj = wv; jj < rows; jj += 4) {
+    const int j = jt * d.TW + jj;
+    const bool in = inner_k && i >= 1 && i <= d.nx && j >= 1 && j <= d.ny;
+    v[(long)c * d.m + i + (long)d.X * (j + (long)d.Y * k)] = in ? t[lane + jj][jj] : 0.0;
+  }
 }
 
 __global__ void k_zero_int(int* p, int n) {
@@ -176,310 +284,449 @@ __global__ void k_zero_int(int* p, int n) {
   if (e < n) p[e] = 0;
 }
 
-// ------------------------------------------------------------------ Gauss-Seidel sweep
-// A sweep is split as the reference's loops are (GaussSeidel_SpDiag :216-234): first
-// t = b - U x_old for every cell (k_gs_upart, fully parallel), then the forward
-// substitution (L+D) x = t (k_gs_lower, the pipelined part).  Term order of a row as in
-// the reference: b, -U (+1, +X, +XY, then JacFall's +XY), -L (-XY, -X, -1), / diag.
+// ------------------------------------------------------------------ Gauss-Seidel sweeps
+// Sweeps one launch runs at most: six wavefronts, the polling and the storing one; two such
+// blocks fit a CU.
+constexpr int kMaxSweeps = 6;
+// Columns of a y-tile at most: a step's values of the top level of a block are five runs of 64
+// (64 columns would take six, and the spare lanes cost less than the extra polls).
+constexpr int kMaxCols = 53;
 constexpr unsigned long long kSentinel = 0xFFF7DEADBEEF0001ull;  // NaN payload: not yet
 
 struct GsArgs {
   Dims d;
-  const double* wmom;  // 7 x sks row coefficients (skewed)
-  const double* wpot;  // 7 x sks
-  const double* wf;    // 2 x sks JacFall rows
-  const double* bs;    // nc x sks right-hand side
-  const double* ts;    // nc x sks right-hand side of the forward substitution
-  double* tw;          // nc x sks: written by k_gs_upart
-  double* xs;          // nc x sks: old values in, new values out
-  double* bnd;         // nc x G x S x Z: last row of each block, for the next block
-  int* counter;        // nc tickets
-  int* err;            // set when a wait gives up
-  int G;
-  int spin_limit;      // polls of a boundary value before a block gives up
-  int hold;            // test hook: no block publishes its last row
+  const double* wmom;   // skewed matrices (k_skew_coef)
+  const double* wpot;
+  const double* wf;     // JacFall rows
+  const double* bs;     // groups x slots x NC: right-hand side
+  const double* ts;     // groups x slots x NC: right-hand side of the first sweep's substitution
+  double* xs;           // groups x slots x NC: result of the last sweep
+  double* bnd;          // groups x [block][step]: boundary records
+  const int* order;     // blocks (jt + NJ*kb) in the order they are taken
+  int* counter;         // ticket
+  int* err;             // set when a wait gives up
+  int NK, M;
+  Groups groups;
+  int nsteps;           // X + TW + KR - 2
+  int spin_limit;       // polls of a boundary value before a block gives up
+  int hold;             // test hook: no block publishes its boundary
 };
 
-// t = b - U x_old on every valid slot (sweeps after the first), all components of a cell
-// in one thread so the U coefficients are read once per cell.
+// t = b - U x_old on every cell (the first sweep of a launch that continues earlier ones).
 template <int NC>
-__global__ __launch_bounds__(256) void k_gs_upart(GsArgs a, Ops ops, int use_mom, int use_pot) {
+__global__ __launch_bounds__(256) void k_gs_upart(GsArgs a, Ops ops, double* __restrict__ tw) {
 #pragma clang fp contract(off)
   const Dims& d = a.d;
-  const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= d.sks) return;
-  const int iz = (int)(k % d.Z);
-  const long t1 = k / d.Z;
-  const int s = (int)(t1 % d.S), iy = (int)(t1 / d.S), ix = s - iz;
-  if (ix < 0 || ix >= d.X) return;
-  const long SZ = (long)d.S * d.Z;
-  const bool ex = ix + 1 < d.X, ey = iy + 1 < d.Y, ez = iz + 1 < d.Z;
-  double up[3] = {0.0, 0.0, 0.0}, um[3] = {0.0, 0.0, 0.0};
-  if (use_pot) {
-    up[0] = a.wpot[4 * d.sks + k], up[1] = a.wpot[5 * d.sks + k], up[2] = a.wpot[6 * d.sks + k];
+  const int lane = threadIdx.x & 63;
+  const int nh = (d.HL + 3) / 4, jt = blockIdx.x / nh;
+  const int h = (blockIdx.x - jt * nh) * 4 + (threadIdx.x >> 6);
+  const int q = blockIdx.z / d.Z, k = blockIdx.z - q * d.Z, g = q / NC, n = q - g * NC;
+  const int c = a.groups.c[g][n];
+  const int j = jt * d.TW + lane, i = h - lane;
+  if (h >= d.HL || lane >= d.TW || j >= d.Y || i < 0 || i >= d.X) return;
+  const long base = g * d.slots * NC + n;
+  const double* const x = a.xs + base;
+  const long row = slot_row(d, jt, h, k), e = row * kRow + lane;
+  const double* const w =
+      (ops.op[c] == ASAM_TR_MOM ? a.wmom : a.wpot) + row * (kCoefWords * kRow) + 2 * lane;
+  double t = a.bs[base + e * NC];
+  if (i + 1 < d.X) t = t - w[coef_word(0)] * x[(e + kRow) * NC];
+  if (j + 1 < d.Y) {
+    // the next column: in this tile one row on, or the first of the next tile, row i
+    const long e2 = lane + 1 < d.TW ? e + kRow + 1 : slot_row(d, jt + 1, i, k) * kRow;
+    t = t - w[coef_word(1)] * x[e2 * NC];
   }
-  if (use_mom) {
-    um[0] = a.wmom[4 * d.sks + k], um[1] = a.wmom[5 * d.sks + k], um[2] = a.wmom[6 * d.sks + k];
+  if (k + 1 < d.Z) {
+    const double xz = x[(e + (long)d.NJ * d.HL * kRow) * NC];
+    t = t - w[coef_word(2)] * xz;
+    if (ops.op[c] == ASAM_TR_FALL)
+      t = t - (a.wf[row * (2 * kRow) + 2 * lane + 1] * ops.alpha[c]) * xz;
   }
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const int op = ops.op[c];
-    const double* w = op == ASAM_TR_MOM ? um : up;
-    const double* __restrict__ x = a.xs + c * d.sks;
-    double t = a.bs[c * d.sks + k];
-    if (ex) t = t - w[0] * x[k + d.Z];
-    if (ey) t = t - w[1] * x[k + SZ];
-    if (ez) {
-      t = t - w[2] * x[k + d.Z + 1];
-      if (op == ASAM_TR_FALL) t = t - (a.wf[d.sks + k] * ops.alpha[c]) * x[k + d.Z + 1];
-    }
-    a.tw[c * d.sks + k] = t;
-  }
+  tw[base + e * NC] = t;
 }
 
-__global__ void k_fill_u64(unsigned long long* p, long n, unsigned long long v) {
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < n) p[e] = v;
+__global__ __launch_bounds__(256) void k_gs_reset(unsigned long long* p, long n,
+                                                  unsigned long long v, int* ticket) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) *ticket = 0;
+  const long e = 2 * ((long)blockIdx.x * blockDim.x + threadIdx.x);
+  if (e + 1 < n) *reinterpret_cast<ulonglong2*>(p + e) = make_ulonglong2(v, v);
+  else if (e < n) p[e] = v;
 }
 
 __device__ __forceinline__ bool is_sentinel(double v) {
-  return (unsigned long long)__double_as_longlong(v) == kSentinel;
+  // no arithmetic gives this payload: the high word is enough
+  return __double2hiint(v) == (int)(kSentinel >> 32);
 }
 
-// Boundary values of C steps for the 128 z-slots of a row, two per lane (z = lane and
-// lane + 64), as one polling wavefront holds them.
-template <int C>
-struct Pend {
-  double v[C][2];
-  bool ok;
-};
+// All sweeps of a preconditioner application in one launch.
+//
+// In the hyperplane order cell (i, j, k) of sweep s can be updated at time T = i + j + k + 2s:
+// its new -x, -y, -z neighbours are done at T - 1, and so are the old +x, +y, +z ones, sweep
+// s - 1 at T - 1.  So the sweeps follow each other two steps apart and the whole application
+// takes X + Y + Z + 2M steps instead of M times X + Y + Z.
+//  - A block owns TW columns j by KR levels k of every sweep and marches along x.  Sweep s of
+//    block (jt, kb) covers columns jt*TW - s + l (lane l) and levels kb*KR - s + r: shifted by
+//    one in both per sweep, so a block needs values of the blocks before it in j and k only.
+//    At the block's step T every sweep is at cell i = T - l - r.
+//  - One wavefront per sweep; a lane computes the KR levels of its column, for NC components
+//    that share their matrix (their coefficients are loaded once).  A step's values pass to
+//    the next step through LDS (double buffered, one barrier per step): the wavefront's own
+//    for the -y neighbour, sweep s - 1's for the old neighbours.  x_old is never read from
+//    memory, and only the last sweep is stored.
+//  - Sweep s reads a cell's coefficients two steps after sweep s - 1, from the caches.  A lane
+//    refills a level's registers for D steps ahead as soon as it has used them.
+//  - A block's top level and last column go to its successors through a record per step,
+//    pre-filled with a NaN-payload sentinel and written and read past the caches that are not
+//    coherent between XCDs: a value that is not the sentinel is final, so no fence or flag
+//    orders them.  One wavefront per block requests the predecessors' values PF steps ahead
+//    and puts them in LDS beside the block's own; one stores the block's.  (A store's
+//    acknowledgement counts like a load's, so a computing wavefront that stored would wait
+//    for it before it could use the loads it issues afterwards.)
+//  - Blocks are taken from an atomic ticket in an order in which a block's predecessors come
+//    first, so a block waits only for blocks that started before it; every wait is bounded.
+//
+// What bounds it: the dependent steps (about 2.1 us each at 256x256x64 with four components: as
+// much for the coefficient loads, 28 cycles of the L1 per 16-byte load of a wavefront, as for
+// the arithmetic, and what the blocks wait for each other's slowest step), and one hand-over of
+// 2.6 us per level block.  256x256x64, four components, 6 sweeps: 1.24 ms; one launch per sweep
+// with a pass for b - U x_old before it, rows handed over along y, took 4.3 ms.  101x77x50,
+// three components: 0.25 ms against 2.1 ms.
+//
+// Term order of a row as in the reference (GaussSeidel_SpDiag :216-234): b, -U (+1, +X, +XY,
+// then JacFall's +XY), -L (-XY, -X, -1), / diag; products and sums are not contracted.  A
+// coupling that leaves the block is +0 and so is the value there, so it changes no sum.
+constexpr int kLdsRow = 66;     // column -1, 64 columns, pad
+constexpr int kZWords = (kMaxSweeps * kMaxCols + 63) / 64;  // runs of 64 in a record's top level
+constexpr int PF = 2;           // steps ahead that a block's boundary values are requested
+constexpr int kSc1 = 16;        // buffer access: to the coherence point of the device
 
-// Re-reads the boundary values that are still the sentinel until every value the first
-// row will use is published; bounded, and kept out of line so that the rare wait does not
-// bloat the kernel's code.  ok = false when it gave up (the error word is then set).
-template <int C>
-__device__ __attribute__((noinline)) Pend<C> settle_boundary(Pend<C> p, const double* bnd_in,
-                                                           int T0, int S, int Z, int X,
-                                                           int limit, int* err) {
-  const int lane = threadIdx.x & 63;
-  int n = 0;
-  p.ok = true;
-  while (true) {
-    bool miss = false;
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+// The values of NC components at one place.
+template <int NC>
+struct alignas(8 * NC) Val {
+  double c[NC];
+};
+template <int NC>
+__device__ __forceinline__ Val<NC> buf_load(__amdgpu_buffer_rsrc_t r, int off) {
+  if constexpr (NC == 1)
+    return __builtin_bit_cast(Val<NC>, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, kSc1));
+  else
+    return __builtin_bit_cast(Val<NC>, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, kSc1));
+}
+template <int NC>
+__device__ __forceinline__ void buf_store(__amdgpu_buffer_rsrc_t r, int off, Val<NC> v) {
+  if constexpr (NC == 1)
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, off, 0, kSc1);
+  else
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, off, 0, kSc1);
+}
+template <int NC>
+__device__ __forceinline__ bool any_sentinel(const Val<NC>& v) {
+  bool m = false;
 #pragma unroll
-    for (int q = 0; q < C; ++q) {
-      const int sl = T0 + q;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int z = lane + 64 * h, ix = sl - z;
-        const bool need = sl >= 0 && sl < S && z < Z && ix >= 0 && ix < X;
-        miss |= need && is_sentinel(p.v[q][h]);
-      }
-    }
-    if (!__any(miss)) return p;
-    if (++n > limit) {
-      __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      p.ok = false;
-      return p;
-    }
-    __builtin_amdgcn_s_sleep(2);
-#pragma unroll
-    for (int q = 0; q < C; ++q) {
-      const int sl = T0 + q;
-      const long o = (long)(sl < 0 ? 0 : (sl >= S ? S - 1 : sl)) * Z;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int z = lane + 64 * h;
-        if (is_sentinel(p.v[q][h]))
-          p.v[q][h] = __hip_atomic_load(bnd_in + o + (z < Z ? z : Z - 1), __ATOMIC_RELAXED,
-                                        __HIP_MEMORY_SCOPE_AGENT);
-      }
-    }
-  }
+  for (int q = 0; q < NC; ++q) m |= is_sentinel(v.c[q]);
+  return m;
 }
 
-// Forward substitution (L+D) x = t, pipelined over rows.  A workgroup is R rows of
-// Q = ceil(Z/64) compute wavefronts (lane iz = 64*qz + lane) plus one polling wavefront;
-// step T of the workgroup is step s = T - j of row j (row iy = g*R + j).
-//  - The steps run in chunks of C.  Each compute wavefront keeps the t and L/D
-//    coefficients of K chunks in registers and refills a chunk's registers as soon as its
-//    steps are done, so the loads of a step are issued (K-1)*C steps before it runs.
-//  - New values of row iy-1 come through LDS (one barrier per step); the z-neighbour from
-//    the lane below (through LDS across the two wavefronts of a row), the x-neighbour
-//    from the lane's own previous step.
-//  - The first row's neighbour row is the previous block's last row.  Its values are
-//    written with agent-scope atomic stores into a buffer pre-filled with a NaN-payload
-//    sentinel; a value that is not the sentinel is final, so no fence or flag orders
-//    them.  The polling wavefront reads them with agent-scope atomic loads, a chunk
-//    ahead and in a wavefront of their own (so no coefficient load is queued ahead of a
-//    poll), and hands them to the first row through LDS.
-//  - Blocks take their rows from an atomic ticket and only wait for a block that started
-//    before them; every wait is bounded.
-template <int C>
-struct Chunk {
-  double t[C], w0[C], w1[C], w2[C], w3[C], f0[C];
-};
-
-constexpr int kBoundStride = 128;  // z-stride of the boundary-value slots in LDS
-
-template <int C, int K, bool FALL>
-__global__ __launch_bounds__(576) void k_gs_lower(GsArgs a, Ops ops, int Q) {
+// DIV: divide by the diagonal (a matrix with an unusual one, or JacFall in it) instead of
+// multiplying by its reciprocal.
+template <int NC, int KR, int D, bool FALL, bool DIV, typename OFF>
+__global__ __launch_bounds__(512, 2) void k_gs_tiles(GsArgs a, Ops ops) {
 #pragma clang fp contract(off)
-  extern __shared__ double lds[];  // [2][R][Z] row exchange, then [2][C][128] boundary values
+  using V = Val<NC>;
+  extern __shared__ __attribute__((aligned(16))) double lds_raw[];
+  V* const lds = reinterpret_cast<V*>(lds_raw);  // [2][M][KR + 1][kLdsRow], level -1, column -1 first
   __shared__ int s_ticket;
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int nw = (blockDim.x >> 6) - 1;  // compute wavefronts; the last one polls
-  const bool poller = wv == nw;
-  const int R = nw / Q;
-  const int j = poller ? 0 : wv / Q, qz = poller ? 0 : wv - j * Q;
   const Dims& d = a.d;
-  const int c = blockIdx.x / a.G;
-  const int op = ops.op[c];
-  // a launch serves the components of one kind (with JacFall or not); the others leave
-  // at once, whole workgroups together, before any barrier
-  if ((op == ASAM_TR_FALL) != FALL) return;
-  if (threadIdx.x == 0) s_ticket = atomicAdd(a.counter + c, 1);
+  const int lane = threadIdx.x & 63, M = a.M, TW = d.TW, X = d.X;
+  const int s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr int kWave = (KR + 1) * kLdsRow;
+  const int half = M * kWave;
+  for (int e = threadIdx.x; e < 2 * half * NC; e += blockDim.x) lds_raw[e] = 0.0;
+  if (threadIdx.x == 0) s_ticket = atomicAdd(a.counter, 1);
   __syncthreads();
-  const int g = s_ticket;
-  const int S = d.S, Z = d.Z, X = d.X;
-  const long SZ = (long)S * Z;
-  const int steps = S + R - 1;
-  // every wavefront runs whole loop turns of K chunks: the steps past `steps` compute
-  // nothing (no cell is valid there), and no branch skips part of a turn, so the
-  // compiler's load-wait counts stay exact across the turn instead of draining
-  const int nchunks = (steps + K * C - 1) / (K * C) * K;
-  double* byL = lds + 2 * R * Z;
-  auto slot = [&](int sl) { return sl < 0 ? 0 : (sl >= S ? S - 1 : sl); };
+  const int ticket = __builtin_amdgcn_readfirstlane(s_ticket);
+  const int g = ticket % a.groups.n, blk = a.order[ticket / a.groups.n];
+  const int jt = blk % d.NJ, kb = blk / d.NJ;
+  const int nsteps = a.nsteps, steps = (nsteps + PF - 1) / PF * PF;
+  // a record: top level [sweep][lane], last column [sweep][level], NC values each
+  const int zrec = M * TW * NC, yrec = M * KR * NC;
+  const long rec = zrec + yrec, brec = nsteps * rec;
+  const long nblk = (long)d.NJ * a.NK;
+  double* const bnd = a.bnd + g * nblk * brec;
 
-  if (poller) {
-    // every barrier of the compute wavefronts is matched here, one per step
-    const bool active = g > 0;
-    const double* bnd_in = a.bnd + ((long)c * a.G + (g > 0 ? g - 1 : 0)) * SZ;
-    Pend<C> p;
-    bool broken = false;
-    auto issue = [&](int T0) {
+  if (s == M) {  // the polling wavefront
+    const int zlast = kb > 0 ? nsteps - 1 - KR : -2;  // values exist up to this time
+    const double* const zrow = bnd + (kb > 0 ? blk - d.NJ : blk) * brec + KR * rec;
+    int zdst[kZWords];
 #pragma unroll
-      for (int q = 0; q < C; ++q) {
-        const long o = (long)slot(T0 + q) * Z;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int z = lane + 64 * h;
-          p.v[q][h] = __hip_atomic_load(bnd_in + o + (z < Z ? z : Z - 1), __ATOMIC_RELAXED,
-                                        __HIP_MEMORY_SCOPE_AGENT);
-        }
-      }
-    };
-    // waits for the values of the chunk at T0 and puts them in LDS slot kc & 1
-    auto settle = [&](int T0, int kc) {
-      bool miss = false;
-#pragma unroll
-      for (int q = 0; q < C; ++q) {
-        const int sl = T0 + q;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int z = lane + 64 * h, ix = sl - z;
-          miss |= sl >= 0 && sl < S && z < Z && ix >= 0 && ix < X && is_sentinel(p.v[q][h]);
-        }
-      }
-      if (__any(miss) && !broken) {
-        p = settle_boundary<C>(p, bnd_in, T0, S, Z, X, a.spin_limit, a.err);
-        broken = !p.ok;
-      }
-#pragma unroll
-      for (int q = 0; q < C; ++q)
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-          byL[((kc & 1) * C + q) * kBoundStride + lane + 64 * h] = p.v[q][h];
-    };
-    if (active) {
-      issue(0);
-      settle(0, 0);
+    for (int q = 0; q < kZWords; ++q) {
+      const int e = lane + 64 * q, w = e / TW;
+      zdst[q] = e < M * TW ? w * kWave + e - w * TW + 1 : kLdsRow - 1;  // or a pad entry
     }
-    __syncthreads();
-    for (int kc = 0; kc < nchunks; ++kc) {
-      const int T0 = kc * C;
+    // the column values, and those of level -1 beside them
+    int f = lane, ylast = -2, ydst = (kLdsRow - 1) * NC;
+    const double* yptr = bnd + blk * brec;
+    if (f < yrec) {
+      const int c = f % NC, e = f / NC, w = e / KR, r = e - w * KR;
+      ydst = (w * kWave + (r + 1) * kLdsRow) * NC + c;
+      if (jt > 0) {
+        yptr = bnd + (blk - 1) * brec + TW * rec + zrec + f;
+        ylast = nsteps - 1 - TW;
+      }
+    } else if ((f -= yrec) < M * NC) {
+      const int c = f % NC, w = f / NC;
+      ydst = w * kWave * NC + c;
+      if (jt > 0 && kb > 0) {
+        yptr = bnd + (blk - d.NJ - 1) * brec + (TW + KR) * rec + (w * TW + TW - 1) * NC + c;
+        ylast = nsteps - 1 - TW - KR;
+      }
+    }
+    struct Poll {
+      V z[kZWords];
+      double y;
+    };
+    bool broken = false;
+    // the values of time th, requested / checked and put in LDS
+    auto issue = [&](int th, Poll& p) {
+      const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<double*>(zrow + (th <= zlast ? th : 0) * rec), 0, zrec * 8, 0x00020000);
 #pragma unroll
-      for (int q = 0; q < C; ++q) {
-        // the next chunk's values: requested after this chunk's first barrier, in LDS
-        // before its last one
-        if (active && q == 0 && T0 + C < steps) issue(T0 + C);
-        if (active && q == C - 1 && T0 + C < steps) settle(T0 + C, kc + 1);
+      for (int q = 0; q < kZWords; ++q) p.z[q] = buf_load<NC>(r, (lane + 64 * q) * (8 * NC));
+      p.y = __hip_atomic_load(yptr + (th <= ylast ? th * rec : 0), __ATOMIC_RELAXED,
+                              __HIP_MEMORY_SCOPE_AGENT);
+    };
+    auto missing = [&](int th, const Poll& p) {
+      bool m = (th <= ylast) & is_sentinel(p.y);
+      if (th <= zlast) {
+#pragma unroll
+        for (int q = 0; q < kZWords; ++q) m |= any_sentinel(p.z[q]);
+      }
+      return __ballot(m) != 0;
+    };
+    auto settle = [&](int th, Poll& p) {
+      if (missing(th, p) && !broken) {
+#pragma clang loop unroll(disable)
+        for (int n = 0;; ++n) {
+          if (n >= a.spin_limit) {
+            __hip_atomic_store(a.err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            broken = true;
+            break;
+          }
+          __builtin_amdgcn_s_sleep(1);
+          issue(th, p);
+          if (!missing(th, p)) break;
+        }
+        // nothing is outstanding here, which the compiler cannot see: without this it would
+        // drain the requests ahead on the common path too
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+      }
+      V* const L = lds + (th & 1) * half;
+#pragma unroll
+      for (int q = 0; q < kZWords; ++q) {
+        V v = p.z[q];
+        if (th > zlast) v = V{};
+        L[zdst[q]] = v;
+      }
+      reinterpret_cast<double*>(L)[ydst] = th <= ylast ? p.y : 0.0;
+    };
+    Poll buf[PF];
+    issue(-1, buf[0]);
+    settle(-1, buf[0]);
+#pragma unroll
+    for (int u = 0; u < PF; ++u) issue(u, buf[u]);
+    __syncthreads();
+    for (int T0 = 0; T0 < steps; T0 += PF) {
+#pragma unroll
+      for (int u = 0; u < PF; ++u) {
+        settle(T0 + u, buf[u]);
+        issue(T0 + u + PF, buf[u]);
         __syncthreads();
       }
     }
     return;
   }
 
-  const int iy = g * R + j;
-  const bool row_ok = iy < d.Y;
-  const double alpha = ops.alpha[c];
-  const double* __restrict__ W = (op == ASAM_TR_MOM) ? a.wmom : a.wpot;
-  const long sks = d.sks;
-  const double* __restrict__ ts = a.ts + c * sks;
-  double* xs = a.xs + c * sks;
-  const long rowbase = (long)(row_ok ? iy : 0) * SZ;
-  const int iz = 64 * qz + lane;
-  const int izc = iz < Z ? iz : Z - 1;
-  const bool publish = j == R - 1 && g + 1 < a.G && row_ok && !a.hold;
-  double* bnd_out = a.bnd + ((long)c * a.G + g) * SZ;
-
-  auto load = [&](int T0, Chunk<C>& ch) {
+  if (s == M + 1) {  // the storing wavefront: the block's records and the last sweep's result
+    const bool pub_z = kb + 1 < a.NK && !a.hold;
+    const bool pub_y = jt + 1 < d.NJ && !a.hold && lane < yrec;
+    int zsrc[kZWords];
 #pragma unroll
-    for (int q = 0; q < C; ++q) {
-      const long k = rowbase + (long)slot(T0 + q - j) * Z + izc;
-      ch.t[q] = ts[k];
-      ch.w0[q] = W[k];
-      ch.w1[q] = W[sks + k];
-      ch.w2[q] = W[2 * sks + k];
-      ch.w3[q] = W[3 * sks + k];
-      ch.f0[q] = FALL ? a.wf[k] : 0.0;
+    for (int q = 0; q < kZWords; ++q) {
+      const int e = lane + 64 * q, w = e / TW;
+      zsrc[q] = e < M * TW ? w * kWave + KR * kLdsRow + e - w * TW + 1 : 0;
     }
-  };
-  double prev = 0.0;
-  // runs the C steps from T0 with coefficients ch, then refills ch with the coefficients
-  // of the chunk K chunks later
-  auto run = [&](int T0, Chunk<C>& ch) {
-    const int kc = T0 / C;
+    const int ye = lane / NC, yw = ye / KR, yr = ye - yw * KR;
+    const int ysrc = pub_y ? (yw * kWave + (yr + 1) * kLdsRow + TW) * NC + lane % NC : 0;
+    double* out = bnd + blk * brec;
+    const int z = M - 1, j = jt * TW - z + lane;
+    const OFF off = ((lane < z ? (OFF)TW : (OFF)d.HL) * kRow + (lane < z ? lane - z + TW : lane - z)) *
+                    (8 * NC);
+    double* const xs = a.xs + g * d.slots * NC;
+    bool cell[KR];
 #pragma unroll
-    for (int q = 0; q < C; ++q) {
-      const int T = T0 + q;
-      const int s = T - j, ix = s - iz;
-      const bool valid = row_ok && s >= 0 && s < S && iz < Z && ix >= 0 && ix < X;
-      const double below = __shfl(prev, (lane + 63) & 63);
-      const int pb = ((T - 1) & 1) * R * Z, cb = (T & 1) * R * Z;
-      // row iy-1: the previous step of row j-1, or for the first row the boundary value
-      double xy_l = 0.0, xz_l = 0.0;
-      if (iz < Z)
-        xy_l = j > 0 ? lds[pb + (j - 1) * Z + iz] : byL[((kc & 1) * C + q) * kBoundStride + iz];
-      if (lane == 0 && qz > 0) xz_l = lds[pb + j * Z + iz - 1];
-      double out = 0.0;
-      if (valid) {
-        double t = ch.t[q];
-        if (iz > 0) t = t - ch.w0[q] * (lane > 0 ? below : xz_l);
-        if (iy > 0) t = t - ch.w1[q] * xy_l;
-        if (ix > 0) t = t - ch.w2[q] * prev;
-        double dg = ch.w3[q];
-        if (FALL) dg = dg + ch.f0[q] * alpha;
-        out = t / dg;
-        xs[rowbase + (long)s * Z + iz] = out;
-        if (publish)
-          __hip_atomic_store(bnd_out + (long)s * Z + iz, out, __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_AGENT);
+    for (int r = 0; r < KR; ++r) {
+      const int k = kb * KR - z + r;
+      cell[r] = (lane < TW) & (j >= 0) & (j < d.Y) & (k >= 0) & (k < d.Z);
+    }
+    __syncthreads();
+    for (int T = 0; T < steps; ++T) {
+      __syncthreads();  // step T is in LDS
+      const V* const L = lds + (T & 1) * half;
+      if (T < nsteps) {
+        if (pub_z) {
+          const __amdgpu_buffer_rsrc_t r =
+              __builtin_amdgcn_make_buffer_rsrc(out, 0, zrec * 8, 0x00020000);
+#pragma unroll
+          for (int q = 0; q < kZWords; ++q)
+            buf_store<NC>(r, (lane + 64 * q) * (8 * NC), L[zsrc[q]]);  // past zrec: dropped
+        }
+        if (pub_y)
+          __hip_atomic_store(out + zrec + lane, reinterpret_cast<const double*>(L)[ysrc],
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        out += rec;
       }
-      if (iz < Z) lds[cb + j * Z + iz] = out;
-      prev = out;
-      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < KR; ++r) {
+        const int k = min(max(kb * KR - z + r, 0), d.Z - 1);
+        char* const row =
+            reinterpret_cast<char*>(xs + slot_row(d, jt - 1, T - r - z, k) * (kRow * NC));
+        if (cell[r] & ((unsigned)(T - lane - r) < (unsigned)X))
+          *reinterpret_cast<V*>(row + off) = L[z * kWave + (r + 1) * kLdsRow + lane + 1];
+      }
     }
-    load(T0 + K * C, ch);
-  };
-  Chunk<C> buf[K];
-#pragma unroll
-  for (int b = 0; b < K; ++b) load(b * C, buf[b]);
-  __syncthreads();  // the first chunk's boundary values are in LDS
-  for (int T0 = 0; T0 < nchunks * C; T0 += K * C) {
-#pragma unroll
-    for (int b = 0; b < K; ++b) run(T0 + b * C, buf[b]);
+    return;
   }
+
+  const int j = jt * TW - s + lane;
+  const int k0 = kb * KR - s;
+  bool col_ok[KR];
+#pragma unroll
+  for (int r = 0; r < KR; ++r)
+    col_ok[r] = (lane < TW) & (j >= 0) & (j < d.Y) & (k0 + r >= 0) & (k0 + r < d.Z);
+  const int op = ops.op[a.groups.c[g][0]];
+  const bool fall = FALL && op == ASAM_TR_FALL;
+  double alpha[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) alpha[c] = FALL ? ops.alpha[a.groups.c[g][c]] : 0.0;
+  const double* const W = op == ASAM_TR_MOM ? a.wmom : a.wpot;
+  const double* const B = (s == 0 ? a.ts : a.bs) + g * d.slots * NC;
+  // Byte offset of the lane's column from row (jt - 1, h) of a level: the columns before the
+  // tile's first lie in tile jt - 1, TW rows on.
+  const OFF rowl = lane < s ? TW : d.HL;
+  const int col = lane < s ? lane - s + TW : lane - s;
+  const OFF offw = (rowl * (kCoefWords * kRow) + 2 * col) * 8, offb = (rowl * kRow + col) * (8 * NC);
+  const OFF offf = (rowl * (2 * kRow) + 2 * col) * 8;
+  // lanes without a cell load the first column of the lane-independent row instead (in the
+  // arrays or their guard rows)
+  const OFF sfw = (OFF)d.HL * (kCoefWords * kRow * 8), sfb = (OFF)d.HL * (kRow * 8 * NC),
+            sff = (OFF)d.HL * (2 * kRow * 8);
+  struct Level {
+    double w[kCoefWords], f0, f1;
+    V b;
+    bool ok;
+  };
+  auto at = [](const double* p, OFF off) { return reinterpret_cast<const char*>(p) + off; };
+  auto load = [&](int T, int r, Level& v) {
+    const bool ok = col_ok[r] & ((unsigned)(T - lane - r) < (unsigned)X);
+    const long row = slot_row(d, jt - 1, T - r - s, min(max(k0 + r, 0), d.Z - 1));
+    const char* const pw = at(W + row * (kCoefWords * kRow), ok ? offw : sfw);
+#pragma unroll
+    for (int q = 0; q < kCoefWords; q += 2) {
+      const double2 x = *reinterpret_cast<const double2*>(pw + coef_word(q) * 8);
+      v.w[q] = x.x;
+      v.w[q + 1] = x.y;
+    }
+    if constexpr (FALL) {
+      const double2 x =
+          *reinterpret_cast<const double2*>(at(a.wf + row * (2 * kRow), ok ? offf : sff));
+      v.f0 = x.x;
+      v.f1 = x.y;
+    }
+    v.b = *reinterpret_cast<const V*>(at(B + row * (kRow * NC), ok ? offb : sfb));
+    v.ok = ok;
+  };
+  Level lv[D][KR];
+  V cur[KR];
+#pragma unroll
+  for (int r = 0; r < KR; ++r) {
+    cur[r] = V{};
+#pragma unroll
+    for (int u = 0; u < D; ++u) load(u, r, lv[u][r]);
+  }
+  __syncthreads();
+  // the steps of a sweep with or without old values (the first one starts from x = 0)
+  auto march = [&](auto old_values) {
+    constexpr bool OLD = decltype(old_values)::value;
+    for (int T0 = 0; T0 < steps; T0 += 2) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const V* const P = lds + ((u + 1) & 1) * half + s * kWave + lane;  // column l - 1
+        const V* const O = P - kWave;                                      // sweep s - 1
+        V* const L = lds + (u & 1) * half + s * kWave + lane + 1;
+        Level(&v)[KR] = lv[u % D];
+        // the chains of all levels and components side by side, without a branch
+        double t[KR][NC], x[KR][NC];
+        bool odd = false;
+#pragma unroll
+        for (int r = 0; r < KR; ++r) {
+          V o0, o1, o2;
+          if constexpr (OLD) {
+            o0 = O[r * kLdsRow];
+            o1 = O[r * kLdsRow + 1];
+            o2 = O[(r + 1) * kLdsRow];
+          }
+          const V below = r == 0 ? P[1] : cur[r > 0 ? r - 1 : 0], west = P[(r + 1) * kLdsRow];
+#pragma unroll
+          for (int c = 0; c < NC; ++c) {
+            double tt = v[r].b.c[c];
+            if constexpr (OLD) {
+              tt = tt - v[r].w[0] * o0.c[c];
+              tt = tt - v[r].w[1] * o1.c[c];
+              tt = tt - v[r].w[2] * o2.c[c];
+              if (FALL && fall) tt = tt - (v[r].f1 * alpha[c]) * o2.c[c];
+            }
+            tt = tt - v[r].w[3] * below.c[c];
+            tt = tt - v[r].w[4] * west.c[c];
+            tt = tt - v[r].w[5] * cur[r].c[c];
+            t[r][c] = tt;
+          }
+        }
+#pragma unroll
+        for (int r = 0; r < KR; ++r) {
+#pragma unroll
+          for (int c = 0; c < NC; ++c) {
+            if constexpr (DIV) {
+              double dg = v[r].w[6];
+              if (FALL && fall) dg = dg + v[r].f0 * alpha[c];
+              x[r][c] = t[r][c] / dg;
+            } else {
+              x[r][c] = gs_divide(t[r][c], v[r].w[6], v[r].w[7]);
+              odd |= gs_odd(x[r][c]) & v[r].ok;
+            }
+          }
+        }
+        if (!DIV && __builtin_expect(__ballot(odd) != 0, 0)) {
+#pragma unroll
+          for (int r = 0; r < KR; ++r)
+#pragma unroll
+            for (int c = 0; c < NC; ++c) x[r][c] = t[r][c] / v[r].w[6];
+        }
+#pragma unroll
+        for (int r = 0; r < KR; ++r) {
+#pragma unroll
+          for (int c = 0; c < NC; ++c) cur[r].c[c] = v[r].ok ? x[r][c] : 0.0;
+          L[(r + 1) * kLdsRow] = cur[r];
+          load(T0 + u + D, r, v[r]);
+        }
+        __syncthreads();
+      }
+    }
+  };
+  if (s > 0) march(std::true_type{});
+  else march(std::false_type{});
 }
 
 // ------------------------------------------------------------------ dots and updates
@@ -541,20 +788,26 @@ struct asam_tr_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   Dims d{};
-  int nc = 0, iterg = 5, M = 1;
+  int nc = 0, iterg = 5;
   Ops ops_mv{}, ops_ps{};  // per-component operator of MatVec and of PSolve
-  asam_tr_tuning tune{8, 2, 0, 0};
+  asam_tr_tuning tune{8, 2, 0, 0};  // gs_rows 4 and more: by size, see sweep_shape
   int hold_boundary = 0;  // test hook (asam_tr_test_hold_boundary)
+  bool odd_diag[2] = {false, false};  // JacTMom, JacTPot: a diagonal gs_divide cannot take
   bool have_mom = false, have_pot = false, have_fall = false, have_lu = false;
   std::string err;
   std::vector<void*> allocs;
   double *tmom = nullptr, *tpot = nullptr, *fall = nullptr, *lu = nullptr;
   double *wmom = nullptr, *wpot = nullptr, *wf = nullptr;
-  double *bs = nullptr, *xs = nullptr, *ts = nullptr, *bnd = nullptr;
+  double *bs = nullptr, *xs = nullptr, *ts = nullptr;
+  double* bnd = nullptr;  // boundary records, grown on demand
+  long bnd_n = 0;
+  int* order = nullptr;   // blocks of the sweeps in the order they are taken, for order_kr
+  int order_kr = 0;
+  std::vector<int> groups;  // sweeps per launch of a preconditioner application
   double *vx = nullptr, *vb = nullptr, *vr = nullptr, *vrt = nullptr, *vrh = nullptr;
   double *vp = nullptr, *vph = nullptr, *vt = nullptr, *vv = nullptr, *vh = nullptr;
   double *partial = nullptr, *dots = nullptr;
-  int *sync = nullptr;  // tickets, error word
+  int *sync = nullptr;  // ticket, error word, set-up flag
   int sync_n = 0;
   double* host_dots = nullptr;  // pinned
 };
@@ -588,17 +841,24 @@ static int tralloc(asam_tr_ctx* c, T** p, size_t count) {
 
 static inline unsigned blocks_for(long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
 
-// Rows per workgroup: at most 8 compute wavefronts (M per row, M = 2 when Z > 64), plus
-// the one that polls the previous block's boundary row.
-static int rows_per_wg(const asam_tr_ctx* c) {
-  int R = c->tune.gs_rows;
-  if (R < 1) R = 1;
-  if (R > 8 / c->M) R = 8 / c->M;
-  return R;
+// Rows of a skewed array in front and behind that lanes without a cell may read.
+constexpr int kGuardRows = 16;
+
+static void trfree(asam_tr_ctx* c, void* p) {
+  for (size_t q = 0; q < c->allocs.size(); ++q)
+    if (c->allocs[q] == p) {
+      c->allocs.erase(c->allocs.begin() + q);
+      break;
+    }
+  (void)hipFree(p);
 }
-static int blocks_y(const asam_tr_ctx* c) {
-  const int R = rows_per_wg(c);
-  return (c->d.Y + R - 1) / R;
+
+// A skewed array of `words` words per slot of n slots, with its guard rows.
+static int skew_alloc(asam_tr_ctx* c, double** p, long n, int words) {
+  const size_t guard = (size_t)kGuardRows * kRow * words * 2;
+  int rc = tralloc(c, p, (size_t)n * words + 2 * guard);
+  if (!rc) *p += guard;
+  return rc;
 }
 
 extern "C" const char* asam_tr_last_error(const asam_tr_ctx* c) {
@@ -615,6 +875,8 @@ extern "C" int asam_tr_destroy(asam_tr_ctx* c) {
   delete c;
   return 0;
 }
+
+static int prepare_sweeps(asam_tr_ctx* c, long places);
 
 extern "C" int asam_tr_create(asam_tr_ctx** out, const asam_tr_grid* g) {
   if (!out || !g) return ASAM_E_INVALID;
@@ -634,13 +896,20 @@ extern "C" int asam_tr_create(asam_tr_ctx** out, const asam_tr_grid* g) {
     return bail(ASAM_E_HIP);
   Dims& d = c->d;
   d.nx = g->nx, d.ny = g->ny, d.nz = g->nz;
-  d.X = (int)X, d.Y = (int)Y, d.Z = (int)Z, d.S = (int)(X + Z - 1);
+  d.X = (int)X, d.Y = (int)Y, d.Z = (int)Z;
   d.m = X * Y * Z;
   d.ncell = (long)g->nx * g->ny * g->nz;
-  d.sks = Y * d.S * Z;
   c->nc = g->ncomp;
   c->iterg = g->iterg;
-  c->M = Z <= 64 ? 1 : 2;
+  // the sweeps of an application in launches of nearly equal size
+  const int total = g->iterg + 1, nl = (total + kMaxSweeps - 1) / kMaxSweeps;
+  for (int q = 0; q < nl; ++q) c->groups.push_back(total / nl + (q < total % nl ? 1 : 0));
+  // y-tiles that cover Y columns at every sweep's shift
+  const int span = d.Y + c->groups[0] - 1;
+  d.NJ = (span + kMaxCols - 1) / kMaxCols;
+  d.TW = (span + d.NJ - 1) / d.NJ;
+  d.HL = d.X + d.TW - 1;
+  d.slots = (long)d.Z * d.NJ * d.HL * kRow;
   c->ops_mv.nc = c->ops_ps.nc = c->nc;
   for (int q = 0; q < kMaxComp; ++q) {
     c->ops_mv.op[q] = c->ops_ps.op[q] = ASAM_TR_POT;
@@ -652,36 +921,34 @@ extern "C" int asam_tr_create(asam_tr_ctx** out, const asam_tr_grid* g) {
   rc |= tralloc(c, &c->tpot, 7 * (size_t)d.m);
   rc |= tralloc(c, &c->fall, 2 * (size_t)d.m);
   rc |= tralloc(c, &c->lu, (size_t)c->nc * c->nc * d.ncell);
-  rc |= tralloc(c, &c->wmom, 7 * (size_t)d.sks);
-  rc |= tralloc(c, &c->wpot, 7 * (size_t)d.sks);
-  rc |= tralloc(c, &c->wf, 2 * (size_t)d.sks);
-  rc |= tralloc(c, &c->bs, (size_t)c->nc * d.sks);
-  rc |= tralloc(c, &c->xs, (size_t)c->nc * d.sks + (size_t)d.S * d.Z + d.Z + 1);
-  rc |= tralloc(c, &c->ts, (size_t)c->nc * d.sks);
-  rc |= tralloc(c, &c->bnd, (size_t)c->nc * d.sks);
+  rc |= skew_alloc(c, &c->wmom, d.slots, kCoefWords);
+  rc |= skew_alloc(c, &c->wpot, d.slots, kCoefWords);
+  rc |= skew_alloc(c, &c->wf, d.slots, 2);
+  // groups of two: room for the places that they repeat, one per operator kind
+  const long places = c->nc == 1 ? 1 : c->nc + std::min(c->nc, 3);
+  rc |= skew_alloc(c, &c->bs, places * d.slots, 1);
+  rc |= skew_alloc(c, &c->xs, places * d.slots, 1);
+  if (c->groups.size() > 1) rc |= skew_alloc(c, &c->ts, places * d.slots, 1);
   double** vecs[] = {&c->vx, &c->vb, &c->vr, &c->vrt, &c->vrh, &c->vp, &c->vph, &c->vt, &c->vv,
                      &c->vh};
   for (double** v : vecs) rc |= tralloc(c, v, V);
   rc |= tralloc(c, &c->partial, 2 * (size_t)kDotBlocks);
   rc |= tralloc(c, &c->dots, 2);
-  c->sync_n = c->nc + 1;  // tickets, error word
+  c->sync_n = 3;  // ticket, error word, set-up flag
   rc |= tralloc(c, &c->sync, (size_t)c->sync_n);
   if (rc) return bail(ASAM_E_NOMEM);
   if (hipHostMalloc((void**)&c->host_dots, 2 * sizeof(double), hipHostMallocDefault) != hipSuccess)
     return bail(ASAM_E_NOMEM);
-  // skewed padding slots must read as 0
-  if (hipMemsetAsync(c->wmom, 0, 7 * sizeof(double) * d.sks, c->stream) != hipSuccess ||
-      hipMemsetAsync(c->wpot, 0, 7 * sizeof(double) * d.sks, c->stream) != hipSuccess ||
-      hipMemsetAsync(c->wf, 0, 2 * sizeof(double) * d.sks, c->stream) != hipSuccess ||
-      hipMemsetAsync(c->xs, 0, sizeof(double) * ((size_t)c->nc * d.sks + (size_t)d.S * d.Z + d.Z + 1),
-                     c->stream) != hipSuccess ||
-      hipMemsetAsync(c->bs, 0, (size_t)c->nc * sizeof(double) * d.sks, c->stream) != hipSuccess ||
-      hipMemsetAsync(c->sync, 0, sizeof(int) * c->sync_n, c->stream) != hipSuccess ||
+  if (hipMemsetAsync(c->sync, 0, sizeof(int) * c->sync_n, c->stream) != hipSuccess ||
       hipStreamSynchronize(c->stream) != hipSuccess)
     return bail(ASAM_E_HIP);
+  if (int e = prepare_sweeps(c, places)) return bail(e);
   *out = c;
   return 0;
 }
+
+// Grid of the kernels that transpose to the skewed layout.
+static dim3 skew_grid(const Dims& d, int levels) { return dim3(d.NJ * h_blocks(d), 1, levels); }
 
 extern "C" int asam_tr_set_matrix(asam_tr_ctx* c, int which, int numdiag, int diag,
                                   const int* ptr, const double* val) {
@@ -707,9 +974,13 @@ extern "C" int asam_tr_set_matrix(asam_tr_ctx* c, int which, int numdiag, int di
     double* w = which == ASAM_TR_JACTMOM ? c->wmom : c->wpot;
     TRCHK(c, hipSetDevice(c->device));
     TRCHK(c, hipMemcpyAsync(dst, val, 7 * sizeof(double) * m, hipMemcpyHostToDevice, c->stream));
-    k_skew_coef<<<blocks_for(m, 256), 256, 0, c->stream>>>(d, dst, w);
+    k_zero_int<<<1, 64, 0, c->stream>>>(c->sync + 2, 1);
+    k_skew_coef<<<skew_grid(d, d.Z), 256, 0, c->stream>>>(d, dst, w, c->sync + 2);
     TRCHK(c, hipGetLastError());
+    int odd = 0;
+    TRCHK(c, hipMemcpyAsync(&odd, c->sync + 2, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     TRCHK(c, hipStreamSynchronize(c->stream));
+    c->odd_diag[which] = odd != 0;
     (which == ASAM_TR_JACTMOM ? c->have_mom : c->have_pot) = true;
     return 0;
   }
@@ -720,7 +991,7 @@ extern "C" int asam_tr_set_matrix(asam_tr_ctx* c, int which, int numdiag, int di
       if (!std::isfinite(val[e])) return trfail(c, ASAM_E_NAN, "non-finite Val");
     TRCHK(c, hipSetDevice(c->device));
     TRCHK(c, hipMemcpyAsync(c->fall, val, 2 * sizeof(double) * m, hipMemcpyHostToDevice, c->stream));
-    k_skew_fall<<<blocks_for(m, 256), 256, 0, c->stream>>>(d, c->fall, c->wf);
+    k_skew_fall<<<skew_grid(d, d.Z), 256, 0, c->stream>>>(d, c->fall, c->wf);
     TRCHK(c, hipGetLastError());
     TRCHK(c, hipStreamSynchronize(c->stream));
     c->have_fall = true;
@@ -804,91 +1075,182 @@ static int launch_matvec(asam_tr_ctx* c, const double* x, double* y, int init) {
   return 0;
 }
 
-template <int C, int K, bool FALL>
-static void lower_launch(asam_tr_ctx* c, const GsArgs& a, int R, int Q) {
-  const size_t lds = (2 * (size_t)R * c->d.Z + 2 * (size_t)C * kBoundStride) * sizeof(double);
-  k_gs_lower<C, K, FALL><<<(unsigned)(c->nc * a.G), 64 * (R * Q + 1), lds, c->stream>>>(
-      a, c->ops_ps, Q);
+template <int NC, int KR, int D, bool FALL, bool DIV>
+static void tiles_launch(asam_tr_ctx* c, const GsArgs& a, unsigned blocks) {
+  const size_t lds = 2 * (size_t)a.M * (KR + 1) * kLdsRow * sizeof(double) * NC;
+  const dim3 threads(64 * (a.M + 2));
+  // 32-bit byte offsets within a tile's rows, except for blocks of about a million cells in x
+  if ((long)(a.d.HL + 1) * (kCoefWords * kRow * 8) < (1L << 32))
+    k_gs_tiles<NC, KR, D, FALL, DIV, unsigned><<<blocks, threads, lds, c->stream>>>(a,
+                                                                                       c->ops_ps);
+  else
+    k_gs_tiles<NC, KR, D, FALL, DIV, unsigned long>
+        <<<blocks, threads, lds, c->stream>>>(a, c->ops_ps);
 }
 
-// gs_chunk 2: chunks of 2 steps, 4 in registers; 4: chunks of 4 steps, 2 in registers
-template <bool FALL>
-static void lower_kind(asam_tr_ctx* c, const GsArgs& a, int R) {
-  if (c->tune.gs_chunk >= 4) lower_launch<4, 2, FALL>(c, a, R, c->M);
-  else lower_launch<2, 4, FALL>(c, a, R, c->M);
+template <int NC, int KR, int D>
+static void tiles_kind(asam_tr_ctx* c, const GsArgs& a, unsigned blocks) {
+  const bool fall = uses(c->ops_ps, c->nc, ASAM_TR_FALL);
+  const bool odd = (uses(c->ops_ps, c->nc, ASAM_TR_MOM) && c->odd_diag[ASAM_TR_JACTMOM]) ||
+                   c->odd_diag[ASAM_TR_JACTPOT];
+  if (fall) tiles_launch<NC, KR, D, true, true>(c, a, blocks);
+  else if (odd) tiles_launch<NC, KR, D, false, true>(c, a, blocks);
+  else tiles_launch<NC, KR, D, false, false>(c, a, blocks);
 }
 
-template <int NC>
-static void upart_nc(asam_tr_ctx* c, const GsArgs& a, int use_mom, int use_pot) {
-  k_gs_upart<NC><<<blocks_for(c->d.sks, 256), 256, 0, c->stream>>>(a, c->ops_ps, use_mom,
-                                                                     use_pot);
-}
-
-static int launch_upart(asam_tr_ctx* c, const GsArgs& a) {
-  int mom = 0, pot = 0;
-  for (int q = 0; q < c->nc; ++q) (c->ops_ps.op[q] == ASAM_TR_MOM ? mom : pot) = 1;
-  switch (c->nc) {
-#define NCCASE(n) \
-  case n:         \
-    upart_nc<n>(c, a, mom, pot); \
-    break;
-    NCCASE(1) NCCASE(2) NCCASE(3) NCCASE(4) NCCASE(5) NCCASE(6) NCCASE(7) NCCASE(8)
-    NCCASE(9) NCCASE(10) NCCASE(11) NCCASE(12) NCCASE(13) NCCASE(14) NCCASE(15) NCCASE(16)
-#undef NCCASE
-    default:
-      return trfail(c, ASAM_E_INVALID, "ncomp");
+// The components in groups of nc_per of the same operator; a group's second place repeats
+// its first when no component is left for it.
+static Groups make_groups(const asam_tr_ctx* c, int nc_per) {
+  Groups g;
+  g.n = 0;
+  int open[3] = {-1, -1, -1};
+  for (int q = 0; q < c->nc; ++q) {
+    int& o = open[c->ops_ps.op[q]];
+    if (nc_per == 2 && o >= 0) {
+      g.c[o][1] = q;
+      o = -1;
+    } else {
+      g.c[g.n][0] = g.c[g.n][1] = q;
+      o = g.n++;
+    }
   }
+  return g;
+}
+
+// Levels per block and components per group of the sweeps: those that the tuning names (1-3
+// levels), or by size.  A block of two levels of one component takes the shortest steps; with
+// up to a block per CU nothing else counts (101x77x50, three components, 174 blocks: 6 sweeps
+// in 249 us, against 325 us with three levels and 331 us with two components).  Beyond that,
+// blocks of three levels and, where components share a matrix, two of them pass the fewest
+// coefficients through the caches per cell (256x256x64, four components: 1238 us, against 1385
+// us and 1311 us for one component with two and three levels, 1672 us for two with two).
+struct Shape {
+  int KR, NC;
+};
+static Shape sweep_shape(const asam_tr_ctx* c) {
+  constexpr int kCus = 256;
+  const int named = c->tune.gs_rows;
+  auto blocks = [&](int KR, int groups) {
+    return (long)groups * c->d.NJ * ((c->d.Z + c->groups[0] - 1 + KR - 1) / KR);
+  };
+  const int KR = named <= 3 ? named : (blocks(2, c->nc) <= kCus ? 2 : 3);
+  const bool pairs = make_groups(c, 2).n < c->nc;
+  return {KR, pairs && blocks(KR, c->nc) > kCus ? 2 : 1};
+}
+
+// The block order for KR levels per block: by the step of the application at which a block
+// starts, which puts its predecessors in j and k before it.
+static int ensure_order(asam_tr_ctx* c, int KR) {
+  if (c->order_kr == KR) return 0;
+  const Dims& d = c->d;
+  const int NK = (d.Z + c->groups[0] - 1 + KR - 1) / KR;
+  std::vector<int> o((size_t)d.NJ * NK);
+  for (size_t q = 0; q < o.size(); ++q) o[q] = (int)q;
+  auto start = [&](int b) { return (long)(b % d.NJ) * d.TW + (long)(b / d.NJ) * KR; };
+  std::stable_sort(o.begin(), o.end(), [&](int x, int y) { return start(x) < start(y); });
+  if (c->order) {
+    TRCHK(c, hipStreamSynchronize(c->stream));
+    trfree(c, c->order);
+    c->order = nullptr;
+    c->order_kr = 0;
+  }
+  if (int rc = tralloc(c, &c->order, o.size())) return rc;
+  TRCHK(c, hipMemcpyAsync(c->order, o.data(), o.size() * sizeof(int), hipMemcpyHostToDevice,
+                          c->stream));
+  TRCHK(c, hipStreamSynchronize(c->stream));
+  c->order_kr = KR;
   return 0;
 }
 
-// One Gauss-Seidel sweep over every component: t = b - U x_old (not for the first
-// sweep, which starts from x = 0), then the pipelined forward substitution.  Tickets are
-// cleared and the boundary rows reset to the sentinel first.
-static int launch_sweep(asam_tr_ctx* c, int sweep) {
+// The boundary records hold at least n doubles.
+static int ensure_records(asam_tr_ctx* c, long n) {
+  if (n <= c->bnd_n) return 0;
+  TRCHK(c, hipStreamSynchronize(c->stream));
+  if (c->bnd) trfree(c, c->bnd);
+  c->bnd = nullptr;
+  c->bnd_n = 0;
+  if (int rc = tralloc(c, &c->bnd, (size_t)n)) return rc;
+  c->bnd_n = n;
+  return 0;
+}
+
+// Blocks, and doubles of their boundary records per component, of M sweeps in blocks of KR
+// levels.
+static long sweep_blocks(const asam_tr_ctx* c, int KR) {
+  return (long)c->d.NJ * ((c->d.Z + c->groups[0] - 1 + KR - 1) / KR);
+}
+static long sweep_records(const asam_tr_ctx* c, int KR, int M) {
+  return sweep_blocks(c, KR) * (c->d.X + c->d.TW + KR - 2) * M * (c->d.TW + KR);
+}
+
+// Block order and boundary records of the default shape, for `places` components.
+static int prepare_sweeps(asam_tr_ctx* c, long places) {
+  const int KR = sweep_shape(c).KR;
+  if (int rc = ensure_order(c, KR)) return rc;
+  return ensure_records(c, places * sweep_records(c, KR, c->groups[0]));
+}
+
+// One launch of M sweeps over every component; first: from x = 0, else from xs.  The ticket
+// is cleared and the boundary records reset to the sentinel first.
+template <int NC>
+static int launch_sweeps(asam_tr_ctx* c, const Groups& gr, int M, bool first) {
   const Dims& d = c->d;
-  const int R = rows_per_wg(c), G = blocks_y(c);
-  bool any_fall = false, any_plain = false;
-  for (int q = 0; q < c->nc; ++q)
-    (c->ops_ps.op[q] == ASAM_TR_FALL ? any_fall : any_plain) = true;
+  const int KR = sweep_shape(c).KR;
+  if (int rc = ensure_order(c, KR)) return rc;
   GsArgs a;
   a.d = d;
   a.wmom = c->wmom, a.wpot = c->wpot, a.wf = c->wf;
-  a.bs = c->bs, a.tw = c->ts, a.xs = c->xs, a.bnd = c->bnd;
-  a.ts = sweep > 0 ? c->ts : c->bs;
+  a.bs = c->bs, a.xs = c->xs;
+  a.ts = first ? c->bs : c->ts;
+  a.order = c->order;
   a.counter = c->sync;
-  a.err = c->sync + c->sync_n - 1;
-  a.G = G;
+  a.err = c->sync + 1;
+  a.NK = (d.Z + c->groups[0] - 1 + KR - 1) / KR;
+  a.M = M;
+  a.groups = gr;
+  a.nsteps = d.X + d.TW + KR - 2;
   a.spin_limit = c->tune.gs_spin_limit > 0 ? c->tune.gs_spin_limit : kSpinLimit;
   a.hold = c->hold_boundary;
-  if (sweep > 0)
-    if (int rc = launch_upart(c, a)) return rc;
-  k_zero_int<<<blocks_for(c->nc, 256), 256, 0, c->stream>>>(c->sync, c->nc);
-  const long nb = (long)c->nc * G * d.S * d.Z;
-  k_fill_u64<<<blocks_for(nb, 256), 256, 0, c->stream>>>((unsigned long long*)c->bnd, nb,
-                                                          kSentinel);
-  if (any_plain) lower_kind<false>(c, a, R);
-  if (any_fall) lower_kind<true>(c, a, R);
+  const long nblk = sweep_blocks(c, KR), nb = gr.n * NC * sweep_records(c, KR, M);
+  if (int rc = ensure_records(c, nb)) return rc;
+  a.bnd = c->bnd;
+  if (!first)
+    k_gs_upart<NC><<<dim3(d.NJ * ((d.HL + 3) / 4), 1, d.Z * gr.n * NC), 256, 0, c->stream>>>(
+        a, c->ops_ps, c->ts);
+  k_gs_reset<<<blocks_for((nb + 1) / 2, 256), 256, 0, c->stream>>>((unsigned long long*)c->bnd, nb,
+                                                                    kSentinel, c->sync);
+  const unsigned blocks = (unsigned)(gr.n * nblk);
+  if (KR == 1) tiles_kind<NC, 1, 2>(c, a, blocks);
+  else if (KR == 2) tiles_kind<NC, 2, NC == 1 ? 2 : 1>(c, a, blocks);
+  else tiles_kind<NC, 3, 1>(c, a, blocks);
+  TRCHK(c, hipGetLastError());
+  return 0;
+}
+
+template <int NC>
+static int psolve_nc(asam_tr_ctx* c, const double* x, double* y) {
+  const Dims& d = c->d;
+  const Groups gr = make_groups(c, NC);
+  const int levels = d.Z * gr.n * NC;
+  k_zero_int<<<1, 64, 0, c->stream>>>(c->sync + 1, 1);
+  k_skew_vec<NC><<<skew_grid(d, levels), 256, 0, c->stream>>>(d, gr, x, c->bs);
+  TRCHK(c, hipGetLastError());
+  for (size_t q = 0; q < c->groups.size(); ++q)
+    if (int rc = launch_sweeps<NC>(c, gr, c->groups[q], q == 0)) return rc;
+  k_unskew<NC><<<dim3(d.NJ * ((d.X + kTileH - 1) / kTileH), 1, levels), 256, 0, c->stream>>>(
+      d, gr, c->xs, y);
   TRCHK(c, hipGetLastError());
   return 0;
 }
 
 // PSolve_Vec4CellSp: y = GS^(1+IterG)(x) per component, halo zero.  x may equal y.
 static int launch_psolve(asam_tr_ctx* c, const double* x, double* y) {
-  const Dims& d = c->d;
-  const long V = (long)c->nc * d.m;
-  k_zero_int<<<1, 64, 0, c->stream>>>(c->sync + c->sync_n - 1, 1);
-  k_skew_vec<<<blocks_for(V, 256), 256, 0, c->stream>>>(d, c->nc, x, c->bs);
-  TRCHK(c, hipGetLastError());
-  for (int sw = 0; sw <= c->iterg; ++sw)
-    if (int rc = launch_sweep(c, sw)) return rc;
-  k_unskew<<<blocks_for(V, 256), 256, 0, c->stream>>>(d, c->nc, c->xs, y);
-  TRCHK(c, hipGetLastError());
-  return 0;
+  return sweep_shape(c).NC == 2 ? psolve_nc<2>(c, x, y) : psolve_nc<1>(c, x, y);
 }
 
 static int check_gs_error(asam_tr_ctx* c) {
   int e = 0;
-  TRCHK(c, hipMemcpyAsync(&e, c->sync + c->sync_n - 1, sizeof(int), hipMemcpyDeviceToHost,
+  TRCHK(c, hipMemcpyAsync(&e, c->sync + 1, sizeof(int), hipMemcpyDeviceToHost,
                           c->stream));
   TRCHK(c, hipStreamSynchronize(c->stream));
   if (e) return trfail(c, ASAM_E_HIP, "Gauss-Seidel sweep: a workgroup waited past its limit");
@@ -1092,9 +1454,6 @@ extern "C" int asam_tr_set_tuning(asam_tr_ctx* c, const asam_tr_tuning* t) {
   if (t->gs_rows < 1 || t->gs_rows > 8) return trfail(c, ASAM_E_INVALID, "gs_rows");
   if (t->gs_chunk != 2 && t->gs_chunk != 4) return trfail(c, ASAM_E_INVALID, "gs_chunk");
   if (t->gs_spin_limit < 0) return trfail(c, ASAM_E_INVALID, "gs_spin_limit");
-  if ((2 * (size_t)t->gs_rows * c->d.Z + 2 * (size_t)t->gs_chunk * kBoundStride) *
-          sizeof(double) > 60 * 1024)
-    return trfail(c, ASAM_E_INVALID, "gs_rows: LDS");
   c->tune = *t;
   return 0;
 }
@@ -1115,7 +1474,8 @@ extern "C" int asam_tr_time_kernel(asam_tr_ctx* c, int which, int reps, double* 
   int rc = 0;
   auto once = [&]() -> int {
     if (which == 0) {
-      TRY(launch_sweep(c, 1));
+      if (sweep_shape(c).NC == 2) TRY(launch_sweeps<2>(c, make_groups(c, 2), c->groups[0], true));
+      else TRY(launch_sweeps<1>(c, make_groups(c, 1), c->groups[0], true));
     } else if (which == 1) {
       TRY(launch_matvec(c, c->vp, c->vv, 0));
     } else {
@@ -1123,11 +1483,9 @@ extern "C" int asam_tr_time_kernel(asam_tr_ctx* c, int which, int reps, double* 
     }
     return 0;
   };
-  if (which == 0) {  // sweeps need a skewed right-hand side
-    k_skew_vec<<<blocks_for((long)c->nc * c->d.m, 256), 256, 0, c->stream>>>(c->d, c->nc, c->vp,
-                                                                              c->bs);
-  }
-  rc = once();
+  if (which == 0) rc = launch_psolve(c, c->vp, c->vph);  // the skewed right-hand side
+  if (!rc)
+    rc = once();
   if (!rc) {
     (void)hipEventRecord(e0, c->stream);
     for (int q = 0; q < reps && !rc; ++q) rc = once();
@@ -1135,7 +1493,7 @@ extern "C" int asam_tr_time_kernel(asam_tr_ctx* c, int which, int reps, double* 
     (void)hipEventSynchronize(e1);
     float t = 0.0f;
     (void)hipEventElapsedTime(&t, e0, e1);
-    *ms = t / reps;
+    *ms = t / reps / (which == 0 ? c->groups[0] : 1);  // 0: per sweep of a launch
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);

@@ -69,11 +69,10 @@ typedef struct {
   int matvecs;    /* operator applications, the initial residual included */
 } asam_tr_info;
 
-/* Launch shapes of the Gauss-Seidel sweep (results do not depend on them). */
+/* Launch shapes of the Gauss-Seidel sweeps (results do not depend on them). */
 typedef struct {
-  int gs_rows;       /* y-rows per workgroup: 1..8 (one wavefront per row; two and at most
-                        4 rows when nz > 62) */
-  int gs_chunk;      /* steps whose coefficients a wavefront loads in one batch: 2 or 4 */
+  int gs_rows;       /* z-levels per workgroup: 1, 2 or 3; 4..8 (default 8): by size */
+  int gs_chunk;      /* 2 or 4; has no effect */
   int gs_spin_limit; /* polls of a boundary value before a block stops waiting for it (the
                         call then returns ASAM_E_HIP); 0: 4194304 */
   int reserved;
