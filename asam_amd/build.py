@@ -17,8 +17,9 @@ CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 BUILD = os.path.join(HERE, "_build")
 LIB = os.path.join(LIBDIR, "libasam_sound.so")
-SOURCES = ["setup.hip", "apply.hip", "line.hip", "blas.hip", "solver.hip", "batch.hip",
-           "project.hip", "transport.hip", "noalloc.hip"]
+SOURCES = ["line_2d.hip", "line_2f.hip", "line_1d.hip", "line_1f.hip", "apply.hip", "batch.hip",
+           "line.hip", "setup.hip", "blas.hip", "solver.hip", "project.hip", "transport.hip",
+           "noalloc.hip"]
 
 
 def hipcc() -> str:

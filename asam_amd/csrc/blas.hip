@@ -56,7 +56,7 @@ __global__ __launch_bounds__(256) void k_bicg_update(long n, VT* __restrict__ x,
   // copy of the state
   __shared__ unsigned long long sk[kTailWords];
   if (fold.kind >= 0) {
-    fold_state_256(fold, sk, threadIdx.x);
+    fold_state<4>(fold, sk, threadIdx.x);
     fold_write(fold, sk, threadIdx.x, 256);
     st = reinterpret_cast<const KState*>(sk);
   }

@@ -6,8 +6,8 @@
 //     MultiTriTB (np1=2): kx,ky,kz (coupling without theta), tx,ty,tz (face theta),
 //                         gz (gravity coupling of the z-face above), vol, dut     = 9 words
 //     The face (c, c+e) of direction e is stored at cell c; wall faces hold 0.
-//   line factors (vertical-line LU of the z-tridiagonal): pl, pt, pw,
-//     np1*np1 words each per cell (2x2 blocks column-major [11,21,12,22]).
+//   line factors (the z-tridiagonal of each vertical line, see k_factor): pl, pt, pw;
+//     pt and pw np1*np1 words per cell (2x2 blocks column-major [11,21,12,22]).
 //   vectors: p(1:np1, nx, ny, nz) as in the reference, component fastest.
 // Every array exists in FP64 and (after set-up) in FP32.
 #pragma once
@@ -40,7 +40,7 @@ struct Tuning {
                           // 2: one cell per thread in band order (each XCD its own bands),
                           // 3: z-march of apply_rows rows per thread
   int apply_wg = 512;     // target workgroups per apply launch
-  int line_window = 0;    // levels per load window of the line solve (1, 4, 8; 0: by type)
+  int line_window = 0;    // levels per load window of the line solve (1, 4, 8; 0: by size)
   int line_lds = 1;       // LDS staging budget of the line solve's forward sweep per
                           // workgroup: 0 none (output vector), 1 default, n >= 2 n KiB
   int apply_xcd = 1;      // remap workgroups so each XCD gets a contiguous range of tiles
@@ -55,19 +55,27 @@ struct Tuning {
   int apply_depth = 1;    // variant 3, FP32 2x2 blocks, two rows: levels of loads ahead (1, 2)
   int line_nt = 2;        // line solve's factor loads (and the vectors it reads once):
                           // 0 plain, 1 nontemporal, 2 nontemporal when the factors of the
-                          // solve's precision exceed kLineNtBytes
+                          // solve's precision exceed line_nt_bytes
 };
 
-// Factor footprint above which the line solve's loads default to nontemporal: below it the
-// factors stay resident in the 256 MB Infinity Cache across solves (measured: FP32 MultiTriT
-// 256x256x64, 50 MB of factors, line 24.8 us plain against 28.6 us nontemporal; FP32
-// MultiTriTB, 201 MB, 64.5 us plain against 58.7 us nontemporal).
-constexpr long kLineNtBytes = 64l << 20;
+// Bytes of factors (of the solve's precision, without the tiles' padding) above which the line
+// solve's loads default to nontemporal.  Below, the factors and the vectors stay in the
+// 256 MB Infinity Cache from one solve to the next and plain loads win; above, the factors
+// only push the vectors out.  Where the line lies depends on how much else an iteration
+// touches per byte of factors.  Measured, BiCGStab solves, us plain / nontemporal:
+//   2x2 FP64      43 MB 576/630    130 MB 2088/2111   176 MB 2973/2980   242 MB 4111/3966
+//   2x2 mixed     22 MB 486/508     88 MB 1690/1760   121 MB 2218/2196   185 MB 3008/2786
+//   1-comp. FP64  25 MB 900/949     48 MB 1387/1492    66 MB 2070/1870   101 MB 2693/2634
+//   1-comp. mixed 24 MB 1072/1106   50 MB 1541/1595    63 MB 2247/2066    94 MB 3213/3118
+constexpr long line_nt_bytes(int np1, int word) {
+  return (np1 == 1 ? 56l : word == 8 ? 176l : 112l) * 1000000;
+}
 
 struct Geom {
   int nx, ny, nz, np1;
   long N;      // cells
   double fa;   // FacAnela
+  int halves;  // wavefronts per tile of the line solve (line_halves)
   Tuning tune;
 };
 
@@ -81,9 +89,22 @@ __host__ __device__ inline long fac_index(const Geom& g, int i, int j, int k) {
   }
   return i + (long)g.nx * (j + (long)g.ny * k);
 }
-// Words per cell of the line solve's lower blocks L_k.  A 2x2 L_k couples level k to the
-// cell below through one face: L_k = (tz, 1)^T (-kz DUT, gz V) of that cell, rank one, so
-// it is stored as the three words (tz, -kz DUT, gz V).
+// Whether the columns of a grid (or of all members of an ensemble) of `tiles` 64-column tiles
+// are eliminated from both ends (Geom::halves = 2), by two wavefronts per tile: up to two
+// tiles per compute unit.  BiCGStab solves, us from the bottom / from both ends (the better
+// window and cache policy of each):
+//   tiles            64        192       291       480         600         1024
+//   2x2 FP64      466/427   600/565   711/690   2112/2124   2696/2790   5222/5231
+//   2x2 mixed     436/389   505/473   578/555   1287/1276   1619/1602   2750/2784
+//   1-comp. FP64  318/293   434/405   491/471   1114/1119   1350/1337   2603/2657
+//   1-comp. mixed 325/295   354/325   394/373    866/846     962/944    1534/1549
+constexpr int line_halves(long tiles) { return tiles <= 512 ? 2 : 1; }
+// Words per cell of the line solve's blocks towards the previous level of the elimination:
+// L_k, and with elimination from both ends U_k from the middle nz/2 up.  A 2x2 block couples two levels through one
+// face and is rank one, so it is stored as three words: L_k = (tz, 1)^T (-kz DUT, gz V) with
+// the face below and the cell below, U_k = (tz, 1)^T (-kz DUT, -gz V) with the face above and
+// the cell above.  With both ends L of the middle level lies in the bottom level's place,
+// which has no use of its own.
 constexpr int lower_words(int np1) { return np1 == 2 ? 3 : 1; }
 // Entries per line-factor array (tiled layout pads x to a multiple of 64).
 inline long fac_cells(const Geom& g) { return ((long)(g.nx + 63) / 64) * 64 * g.ny * g.nz; }

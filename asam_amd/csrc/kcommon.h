@@ -167,52 +167,62 @@ __device__ __forceinline__ void tail_arrive(const KTail& t, int tid) {
 // (the exit test and beta) reads src, a copy of the state that no workgroup of the launch
 // writes.
 //
-// One wavefront of 64 threads: virtual thread v = 64 w + lane of k_finalize's 1024, the
-// 16 wave totals added in order.
-__device__ __forceinline__ void fold_state_w64(const KTail& f, unsigned long long* sk) {
-  const int lane = threadIdx.x & 63;
+// A workgroup of NW wavefronts: wavefront h adds up the groups w = h, h + NW, ... of
+// k_finalize's 16 (virtual threads 64 w + lane), the group totals are added in order.  Groups
+// without partial sums are skipped: a small grid's step waits for one round trip to memory
+// and a butterfly or two.
+template <int NW>
+__device__ __forceinline__ void fold_state(const KTail& f, unsigned long long* sk, int tid) {
+  __shared__ double sh[4][16];
+  const int lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const KState* src = f.src ? f.src : f.st;
-  for (int w = lane; w < kTailWords; w += 64)
+  for (int w = tid; w < kTailWords; w += 64 * NW)
     sk[w] = reinterpret_cast<const unsigned long long*>(src)[w];
-  double S[4];
+  constexpr int G = 16 / NW < 4 ? 16 / NW : 4;  // groups whose loads are issued together
+  for (int w0 = wid; w0 < 16; w0 += G * NW) {
+    double x[4][G];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    S[q] = 0.0;
-    if (q >= f.nq || !((f.qmask >> q) & 1)) continue;  // uniform
-    const int nb = q < 2 ? f.nblk : f.nblk_hi;
-    const double* pq = f.partial + (long)q * kRedBlocks;
-    // every load of a round unconditional (a clamped index, the value selected after), so
-    // the 16 are in flight together; adding +0.0 for a missing partial keeps the bits
-    double vw[16];
+    for (int q = 0; q < 4; ++q) {
 #pragma unroll
-    for (int w = 0; w < 16; ++w) vw[w] = 0.0;
-    const int rounds = (nb + 1023) >> 10;
-    for (int r = 0; r < rounds; ++r) {
-      double x[16];
+      for (int e = 0; e < G; ++e) x[q][e] = 0.0;
+      const int nb = q < 2 ? f.nblk : f.nblk_hi;
+      if (q >= f.nq || !((f.qmask >> q) & 1) || (w0 << 6) >= nb) continue;  // uniform
+      const double* pq = f.partial + (long)q * kRedBlocks;
+      for (int r = 0; r < nb; r += 1024) {
+        // unconditional loads (a clamped index, the value selected after): adding +0.0 for a
+        // missing partial keeps the bits
+        double y[G];
 #pragma unroll
-      for (int w = 0; w < 16; ++w) x[w] = pq[min((r << 10) + (w << 6) + lane, nb - 1)];
+        for (int e = 0; e < G; ++e) y[e] = pq[min(r + ((w0 + e * NW) << 6) + lane, nb - 1)];
 #pragma unroll
-      for (int w = 0; w < 16; ++w) vw[w] += ((r << 10) + (w << 6) + lane < nb) ? x[w] : 0.0;
+        for (int e = 0; e < G; ++e) x[q][e] += r + ((w0 + e * NW) << 6) + lane < nb ? y[e] : 0.0;
+      }
     }
-    double s = 0.0;
 #pragma unroll
-    for (int w = 0; w < 16; ++w) s += wave_sum(vw[w]);
-    S[q] = s;
+    for (int q = 0; q < 4; ++q) {
+      if (q >= f.nq || !((f.qmask >> q) & 1)) continue;
+      const int nb = q < 2 ? f.nblk : f.nblk_hi;
+#pragma unroll
+      for (int e = 0; e < G; ++e) {
+        const int w = w0 + e * NW;
+        double s = 0.0;
+        if ((w << 6) < nb) s = wave_sum(x[q][e]);
+        if (lane == 0) sh[q][w] = s;
+      }
+    }
   }
   __syncthreads();
-  if (lane == 0) fin_logic(f.kind, S, reinterpret_cast<KState*>(sk), 0, 0, f.nq, nullptr);
-  __syncthreads();
-}
-
-// The same for a workgroup of 256 threads.
-__device__ __forceinline__ void fold_state_256(const KTail& f, unsigned long long* sk, int tid) {
-  const KState* src = f.src ? f.src : f.st;
-  for (int w = tid; w < kTailWords; w += 256)
-    sk[w] = reinterpret_cast<const unsigned long long*>(src)[w];
-  double S[4];
-  tail_sums_256(f, tid, S);
-  __syncthreads();
-  if (tid == 0) fin_logic(f.kind, S, reinterpret_cast<KState*>(sk), 0, 0, f.nq, nullptr);
+  if (tid == 0) {
+    double S[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      S[q] = 0.0;
+      if (q >= f.nq || !((f.qmask >> q) & 1)) continue;
+      const int ng = min(16, ((q < 2 ? f.nblk : f.nblk_hi) + 63) >> 6);
+      for (int w = 0; w < ng; ++w) S[q] += sh[q][w];
+    }
+    fin_logic(f.kind, S, reinterpret_cast<KState*>(sk), 0, 0, f.nq, nullptr);
+  }
   __syncthreads();
 }
 

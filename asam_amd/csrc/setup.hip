@@ -145,9 +145,11 @@ void launch_coef(hipStream_t s, const Geom& g, int grad_full, double beta0_dt, d
 
 // ----------------------------------------------------------- line factorisation
 // LU of each vertical line (Solve_1D, TriDiagT_Mod.f90:135-155; block form with
-// Div_22/Mult_22, TriDiagTB_Mod.f90:143-163):  t_0 = d_0,  w_k-1 = t_k-1^-1 u_k-1,
-// t_k = d_k - l_k-1 w_k-1.  Stored per level k: pl = l_k-1 (0 at k=0),
-// pt = t_k^-1 (0 for a singular t: a dead cell), pw = w_k (0 at the top).
+// Div_22/Mult_22, TriDiagTB_Mod.f90:143-163): t_k = d_k - l_k w_k-1, w_k = t_k^-1 u_k from the
+// bottom to the top.  With elimination from both ends (g.halves = 2) that holds below the
+// middle level m; above it t_k = d_k - u_k w_k+1, w_k = t_k^-1 l_k from the top down, and
+// at m both terms and w_m = 0.  Stored per level k: pl = l_k (u_k from m up; see lower_words),
+// pt = t_k^-1 (0 for a singular t: a dead cell), pw = w_k.
 __device__ __forceinline__ void inv22(const double* m, double* r) {
   double det = m[0] * m[3] - m[2] * m[1];
   if (det == 0.0) { r[0] = r[1] = r[2] = r[3] = 0.0; return; }
@@ -161,105 +163,139 @@ __device__ __forceinline__ void mul22(const double* a, const double* b, double* 
   r[0] = t0; r[1] = t1; r[2] = t2; r[3] = t3;
 }
 
-__global__ void k_factor(Geom g, Coef<double> c) {
-  const int nx = g.nx, ny = g.ny, nz = g.nz;
-  long col = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (col >= (long)nx * ny) return;
-  const int i = col % nx, j = col / nx;
-  const long sy = nx, sz = (long)nx * ny;
-  if (g.np1 == 1) {
-    double t = 0.0, wprev = 0.0;
-    for (int k = 0; k < nz; ++k) {
-      long cc = col + sz * k;
-      const double dut = c.dut[cc];
-      double d = g.fa * c.vol[cc];
-      if (i > 0) d += c.kx[cc - 1] * dut;
-      if (i + 1 < nx) d += c.kx[cc] * dut;
-      if (j > 0) d += c.ky[cc - sy] * dut;
-      if (j + 1 < ny) d += c.ky[cc] * dut;
-      if (k > 0) d += c.kz[cc - sz] * dut;
-      if (k + 1 < nz) d += c.kz[cc] * dut;
-      double l = (k > 0) ? -c.kz[cc - sz] * c.dut[cc - sz] : 0.0;  // row k, col k-1
-      t = (k == 0) ? d : d - l * wprev;
-      double tinv = (t == 0.0) ? 0.0 : 1.0 / t;
-      double w = 0.0;
-      if (k + 1 < nz) {
-        double u = -c.kz[cc] * c.dut[cc + sz];  // row k, col k+1
-        w = (t == 0.0) ? 0.0 : u / t;
-      }
-      const long fi = fac_index(g, i, j, k);
-      c.pl[fi] = l;
-      c.pt[fi] = tinv;
-      c.pw[fi] = w;
-      wprev = w;
+// The blocks of level k of a column: diagonal D, L towards k - 1 and U towards k + 1 (zero past
+// the ends), as l3/u3 in the three words of lower_words.
+struct LineBlocks {
+  double D[4], L[4], U[4], l3[3], u3[3];
+};
+__device__ __forceinline__ LineBlocks line_blocks_at(const Geom& g, const Coef<double>& c, int i,
+                                                     int j, int k) {
+  const long sy = g.nx, sz = (long)g.nx * g.ny, cc = i + sy * j + sz * k;
+  const double dut = c.dut[cc], V = c.vol[cc];
+  LineBlocks b{};
+  auto face = [&](double kk, double th) {
+    if (g.np1 == 1) {
+      b.D[0] += kk * dut;
+    } else {
+      b.D[0] += th * kk * dut;
+      b.D[1] += kk * dut;
     }
-  } else {
-    double W[4] = {0, 0, 0, 0};
-    for (int k = 0; k < nz; ++k) {
-      long cc = col + sz * k;
-      const double dut = c.dut[cc], V = c.vol[cc];
-      double d[4];
-      d[0] = g.fa * V; d[1] = 0.0; d[2] = 0.0; d[3] = V;
-      auto hface = [&](double kk, double th) { d[0] += th * kk * dut; d[1] += kk * dut; };
-      if (i > 0) hface(c.kx[cc - 1], c.tx[cc - 1]);
-      if (i + 1 < nx) hface(c.kx[cc], c.tx[cc]);
-      if (j > 0) hface(c.ky[cc - sy], c.ty[cc - sy]);
-      if (j + 1 < ny) hface(c.ky[cc], c.ty[cc]);
-      double L[4] = {0, 0, 0, 0};
-      double lz_tz = 0.0;  // tz of the face below (L's first row is tz times its second)
-      if (k > 0) {
-        const long m = cc - sz;
-        const double kz = c.kz[m], tz = c.tz[m], gz = c.gz[m];
-        lz_tz = tz;
-        hface(kz, tz);
-        d[2] += tz * gz * V;   // +th g~ V_c   (d(1,2) of the upper cell)
-        d[3] += gz * V;
-        L[0] = -tz * kz * c.dut[m];
-        L[1] = -kz * c.dut[m];
-        L[2] = tz * gz * c.vol[m];
-        L[3] = gz * c.vol[m];
-      }
-      double U[4] = {0, 0, 0, 0};
-      if (k + 1 < nz) {
-        const double kz = c.kz[cc], tz = c.tz[cc], gz = c.gz[cc];
-        hface(kz, tz);
-        d[2] -= tz * gz * V;
-        d[3] -= gz * V;
-        const long p = cc + sz;
-        U[0] = -tz * kz * c.dut[p];
-        U[1] = -kz * c.dut[p];
-        U[2] = -tz * gz * c.vol[p];
-        U[3] = -gz * c.vol[p];
-      }
-      double t[4];
-      if (k == 0) {
-        t[0] = d[0]; t[1] = d[1]; t[2] = d[2]; t[3] = d[3];
-      } else {
-        double LW[4];
-        mul22(L, W, LW);
-        for (int q = 0; q < 4; ++q) t[q] = d[q] - LW[q];
-      }
-      double T[4];
-      inv22(t, T);
-      double Wn[4] = {0, 0, 0, 0};
-      if (k + 1 < nz) mul22(T, U, Wn);
-      const long fi = fac_index(g, i, j, k);
-      for (int q = 0; q < 4; ++q) {
-        c.pt[4 * fi + q] = T[q];
-        c.pw[4 * fi + q] = Wn[q];
-        W[q] = Wn[q];
-      }
-      // L = (tz, 1)^T (L[1], L[3]): the sweeps use the three words
-      c.pl[3 * fi + 0] = lz_tz;
-      c.pl[3 * fi + 1] = L[1];
-      c.pl[3 * fi + 2] = L[3];
+  };
+  const bool two = g.np1 == 2;
+  b.D[0] = g.fa * V;
+  b.D[3] = V;
+  if (i > 0) face(c.kx[cc - 1], two ? c.tx[cc - 1] : 0.0);
+  if (i + 1 < g.nx) face(c.kx[cc], two ? c.tx[cc] : 0.0);
+  if (j > 0) face(c.ky[cc - sy], two ? c.ty[cc - sy] : 0.0);
+  if (j + 1 < g.ny) face(c.ky[cc], two ? c.ty[cc] : 0.0);
+  if (k > 0) {
+    const long m = cc - sz;
+    const double kz = c.kz[m];
+    if (two) {
+      const double tz = c.tz[m], gz = c.gz[m];
+      face(kz, tz);
+      b.D[2] += tz * gz * V;  // +th g~ V_c   (d(1,2) of the upper cell)
+      b.D[3] += gz * V;
+      b.L[0] = -tz * kz * c.dut[m];
+      b.L[1] = -kz * c.dut[m];
+      b.L[2] = tz * gz * c.vol[m];
+      b.L[3] = gz * c.vol[m];
+      b.l3[0] = tz;
+      b.l3[1] = b.L[1];
+      b.l3[2] = b.L[3];
+    } else {
+      face(kz, 0.0);
+      b.l3[0] = b.L[0] = -kz * c.dut[m];
     }
   }
+  if (k + 1 < g.nz) {
+    const long p = cc + sz;
+    const double kz = c.kz[cc];
+    if (two) {
+      const double tz = c.tz[cc], gz = c.gz[cc];
+      face(kz, tz);
+      b.D[2] -= tz * gz * V;
+      b.D[3] -= gz * V;
+      b.U[0] = -tz * kz * c.dut[p];
+      b.U[1] = -kz * c.dut[p];
+      b.U[2] = -tz * gz * c.vol[p];
+      b.U[3] = -gz * c.vol[p];
+      b.u3[0] = tz;
+      b.u3[1] = b.U[1];
+      b.u3[2] = b.U[3];
+    } else {
+      face(kz, 0.0);
+      b.u3[0] = b.U[0] = -kz * c.dut[p];
+    }
+  }
+  return b;
+}
+
+// 64 columns per workgroup, one wavefront for each half; the upper one does the middle level
+// when the lower one has left its last w in LDS.
+__global__ __launch_bounds__(128) void k_factor(Geom g, Coef<double> c) {
+  __shared__ double wl[4][64];
+  const int lane = threadIdx.x & 63, half = threadIdx.x >> 6;
+  const long col = blockIdx.x * 64L + lane;
+  const bool on = col < (long)g.nx * g.ny;
+  const int i = on ? (int)(col % g.nx) : 0, j = on ? (int)(col / g.nx) : 0;
+  const int nz = g.nz, mid = g.halves == 2 ? nz / 2 : nz;
+  double W[4] = {0, 0, 0, 0};
+  // level k: t = D - (block towards the previous level) W [- L_m (lower half's W)]
+  auto level = [&](int k, bool meets) {
+    const LineBlocks b = line_blocks_at(g, c, i, j, k);
+    const double* const A = half ? b.U : b.L;   // towards the previous level
+    const double* const N = half ? b.L : b.U;   // towards the next one
+    const long fi = fac_index(g, i, j, k);
+    if (g.np1 == 1) {
+      double t = b.D[0] - A[0] * W[0];
+      if (meets) t -= b.L[0] * wl[0][lane];
+      const double ti = t == 0.0 ? 0.0 : 1.0 / t;
+      W[0] = meets || t == 0.0 ? 0.0 : N[0] / t;
+      c.pt[fi] = ti;
+      c.pw[fi] = W[0];
+      if (half || k > 0) c.pl[fi] = half ? b.u3[0] : b.l3[0];
+      if (meets && mid > 0) c.pl[fac_index(g, i, j, 0)] = b.l3[0];
+      return;
+    }
+    double t[4], P[4], T[4];
+    mul22(A, W, P);
+    for (int q = 0; q < 4; ++q) t[q] = b.D[q] - P[q];
+    if (meets) {
+      const double w0[4] = {wl[0][lane], wl[1][lane], wl[2][lane], wl[3][lane]};
+      mul22(b.L, w0, P);
+      for (int q = 0; q < 4; ++q) t[q] -= P[q];
+    }
+    inv22(t, T);
+    if (meets) W[0] = W[1] = W[2] = W[3] = 0.0;
+    else mul22(T, N, W);
+    for (int q = 0; q < 4; q += 2) {
+      *reinterpret_cast<double2*>(c.pt + 4 * fi + q) = make_double2(T[q], T[q + 1]);
+      *reinterpret_cast<double2*>(c.pw + 4 * fi + q) = make_double2(W[q], W[q + 1]);
+    }
+    if (half || k > 0)
+      for (int q = 0; q < 3; ++q) c.pl[3 * fi + q] = half ? b.u3[q] : b.l3[q];
+    if (meets && mid > 0) {
+      const long f0 = fac_index(g, i, j, 0);
+      for (int q = 0; q < 3; ++q) c.pl[3 * f0 + q] = b.l3[q];
+    }
+  };
+  if (on) {
+    if (half == 0)
+      for (int k = 0; k < mid; ++k) level(k, false);
+    else
+      for (int k = nz - 1; k > mid; --k) level(k, false);
+  }
+  if (g.halves == 1) return;
+  if (half == 0)
+    for (int q = 0; q < 4; ++q) wl[q][lane] = W[q];
+  __syncthreads();
+  if (on && half) level(mid, true);
 }
 
 void launch_factor(hipStream_t s, const Geom& g, Coef<double>& c) {
   long ncol = (long)g.nx * g.ny;
-  hipLaunchKernelGGL(k_factor, dim3((ncol + 63) / 64), dim3(64), 0, s, g, c);
+  hipLaunchKernelGGL(k_factor, dim3((ncol + 63) / 64), dim3(64 * g.halves), 0, s, g, c);
 }
 
 __global__ void k_cvt(long n, const double* a, float* b) {

@@ -207,6 +207,7 @@ extern "C" int asam_sound_create(asam_sound_ctx** out, const asam_sound_grid* gr
   asam_sound_default_control(&c->ctl);
   c->g.nx = grid->nx; c->g.ny = grid->ny; c->g.nz = grid->nz; c->g.np1 = grid->np1;
   c->g.N = N; c->g.fa = grid->fac_anela;
+  c->g.halves = line_halves(line_blocks(c->g));
   c->n = N * grid->np1;
   int rc = 0;
   auto fin = [&](int code) { *out = c; return code; };
