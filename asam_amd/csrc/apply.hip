@@ -8,13 +8,15 @@
 // columns per wavefront (coalesced along x at every level), loads issued a window of
 // levels ahead of the recurrence, forward-sweep results staged in LDS for the
 // backward sweep.
+#include <algorithm>
+
 #include "asam_sound.h"
 #include "apply_tile.h"
 
 namespace asam {
 
 struct ApplyShape {
-  int gx, gy, kp, ntiles, nblocks;
+  int bx, gx, gy, kp, ntiles, nblocks;
 };
 
 // Rows per band of the band-ordered variant: the tuning's value, or ny/8 rounded up so that
@@ -26,39 +28,91 @@ static int band_rows(const Geom& g) {
   return rb;
 }
 
-// Variants 0, 1 and 3: tiles of bx x (256/bx) columns (variant 3: x apply_rows rows per
-// thread) by kp planes, at most ~apply_wg
-// workgroups, padded to a multiple of the 8 XCDs so that the physical -> logical remap below
-// is a bijection.  Variant 2: apply_wg workgroups (a multiple of 8) looping over the tiles
-// of their XCD's bands.
-static ApplyShape apply_shape(const Geom& g, int fp32) {
+// Tiles of bx columns by `rows` rows by kp planes, padded to a multiple of the 8 XCDs so that
+// the physical -> logical remap of the kernels is a bijection.
+static ApplyShape tile_shape(const Geom& g, int bx, int rows, int kp) {
   ApplyShape a;
-  const int bxw = g.tune.apply_bx, byw = 256 / bxw;
-  a.gx = (g.nx + bxw - 1) / bxw;
-  if (g.tune.apply_variant == 2) {
+  a.bx = bx;
+  a.gx = (g.nx + bx - 1) / bx;
+  a.gy = (g.ny + rows - 1) / rows;
+  a.kp = kp;
+  a.ntiles = (int)((long)a.gx * a.gy * ((g.nz + kp - 1) / kp));
+  a.nblocks = ((a.ntiles + 7) / 8) * 8;
+  return a;
+}
+
+// The default shape (variant 3, two rows per thread): the launch ends with the compute unit
+// that has most to do, so take the tile for which that is least.  A unit with n tiles of kp
+// planes takes n (kp + 1) plane times: kp + 1 because a tile starts by loading the planes
+// around its first one; n no less than the tiles a unit needs at once to be busy, two, and
+// three for one component in FP32, which moves the fewest bytes.  A plane time is the
+// wavefronts of the tile that have columns at all; 32 columns (two stacked row blocks per
+// wavefront) cost a tenth more.  Against 128 columns and about 512 workgroups for every grid,
+// BiCGStab solves, us before / after: 201x150x50 one component FP64 1360/1201, 2x2 FP64
+// 2790/2480, 2x2 mixed 1638/1454; 256x192x56 2x2 FP64 4132/3714, one component mixed
+// 1259/1160; 301x280x60 2x2 FP64 8202/7382, one component FP64 4321/3826; 130x97x40 2x2
+// mixed 579/510; 512x512x96 one component mixed 9118/8518; 256x256x64 2x2: the same shape.
+static ApplyShape balanced_shape(const Geom& g, int fp32) {
+  constexpr int kCUs = 256;
+  const int busy = g.np1 == 1 && fp32 ? 3 : 2;
+  ApplyShape best{};
+  long least = 0;
+  for (int bx : {128, 256, 64, 32}) {
+    const int rows = 256 / bx * 2;
+    const long cols = (long)((g.nx + bx - 1) / bx) * ((g.ny + rows - 1) / rows);
+    const int waves = g.nx < bx ? (g.nx + 63) / 64 * (bx < 64 ? 4 : 256 / bx) : 4;
+    int last = 0;
+    for (int n = 1; n <= 8; ++n) {
+      const long nzt = n * kCUs / cols;
+      const int kp = nzt < 1 ? g.nz : nzt >= g.nz ? 1 : (int)((g.nz + nzt - 1) / nzt);
+      if (kp == last) continue;
+      last = kp;
+      const ApplyShape a = tile_shape(g, bx, rows, kp);
+      const long per = std::max((a.nblocks + kCUs - 1) / kCUs, busy);
+      const long cost = per * waves * (kp + 1) * (bx == 32 ? 11 : 10);
+      if (a.nblocks <= kRedBlocks && (least == 0 || cost < least)) {
+        least = cost;
+        best = a;
+      }
+    }
+  }
+  return best;
+}
+
+// Variants 0, 1 and 3: tiles of bx x (256/bx) columns (variant 3: x apply_rows rows per
+// thread) by kp planes, at most ~apply_wg workgroups.  At the default variant and size of the
+// tuning the shape follows the grid (balanced_shape).  Variant 2: apply_wg workgroups (a
+// multiple of 8) looping over the tiles of their XCD's bands.
+static ApplyShape apply_shape(const Geom& g, int fp32) {
+  const Tuning& t = g.tune;
+  const int bxw = t.apply_bx, byw = 256 / bxw;
+  if (t.apply_variant == 2) {
     const int rb = band_rows(g);
+    ApplyShape a;
+    a.bx = bxw;
+    a.gx = (g.nx + bxw - 1) / bxw;
     a.gy = (rb + byw - 1) / byw;  // row tiles per band
     a.kp = 1;
     a.ntiles = 0;
-    int nb = (g.tune.apply_wg / 8) * 8;
+    int nb = (t.apply_wg / 8) * 8;
     if (nb < 8) nb = 8;
     a.nblocks = nb;
     return a;
   }
+  if (t.apply_variant == 3 && t.apply_rows == 2 && t.apply_wg == 512 && bxw == 128 &&
+      t.apply_xcd) {
+    const ApplyShape a = balanced_shape(g, fp32);
+    if (a.nblocks > 0) return a;
+  }
   // variant 3 tiles: four rows per thread with FP32 coefficients only (see apply_t)
-  const int rpt = (g.tune.apply_variant == 3 && g.tune.apply_rows == 4 && fp32) ? 4 : 2;
-  const int rows = g.tune.apply_variant == 3 ? byw * rpt : byw;
-  a.gy = (g.ny + rows - 1) / rows;
-  long cols = (long)a.gx * a.gy;
-  long want = g.tune.apply_wg;
+  const int rpt = (t.apply_variant == 3 && t.apply_rows == 4 && fp32) ? 4 : 2;
+  const int rows = t.apply_variant == 3 ? byw * rpt : byw;
+  const long cols = (long)((g.nx + bxw - 1) / bxw) * ((g.ny + rows - 1) / rows);
+  const long want = t.apply_wg;
   int kp = (int)((cols * g.nz + want - 1) / want);
   if (kp < 1) kp = 1;
   if (kp > g.nz) kp = g.nz;
-  a.kp = kp;
-  int nzt = (g.nz + kp - 1) / kp;
-  a.ntiles = (int)(cols * nzt);
-  a.nblocks = ((a.ntiles + 7) / 8) * 8;
-  return a;
+  return tile_shape(g, bxw, rows, kp);
 }
 
 int apply_blocks(const Geom& g, int fp32) { return apply_shape(g, fp32).nblocks; }
@@ -321,7 +375,7 @@ static void apply_t(hipStream_t s, const Geom& g, const Coef<CT>& c, const Apply
   a.c = c; a.nx = g.nx; a.ny = g.ny; a.nz = g.nz; a.fa = (CT)g.fa;
   ApplyShape sh = apply_shape(g, sizeof(CT) == 4 ? 1 : 0);
   a.gx = sh.gx; a.gy = sh.gy; a.kp = sh.kp; a.ntiles = sh.ntiles;
-  a.bxw = g.tune.apply_bx; a.byw = 256 / g.tune.apply_bx; a.xcd = g.tune.apply_xcd;
+  a.bxw = sh.bx; a.byw = 256 / sh.bx; a.xcd = g.tune.apply_xcd;
   a.x = (const VX*)r.x; a.dx = r.dx; a.xw = r.xw; a.b = r.b; a.y = (VO*)r.y;
   a.y2 = (VO*)r.y2; a.u = (const VU*)r.u; a.partial = r.partial; a.done = r.done;
   a.dead = r.x0_dead;

@@ -337,6 +337,7 @@ struct asam_ens_ctx {
   long pstride = 0, pcap = 0;
   int *tA = nullptr, *tL = nullptr, *tB = nullptr;
   int halves = 1;  // wavefronts per tile of the line solve, by the tiles of all members
+  int abx = 256;   // columns per apply tile
   int nA = 0, nL = 0, nB = 0;
   long capA = 0, capL = 0, capB = 0;
   EnsMember* md = nullptr;
@@ -456,15 +457,40 @@ static int valid_tuning(const asam_ens_tuning& t) {
 
 // Tile tables of the current tuning (device copies), partial-sum stride.
 static int build_tables(asam_ens_ctx* c) {
-  const int bx = c->tune.apply_bx, chunk = c->tune.blas_chunk;
+  const int chunk = c->tune.blas_chunk;
+  // At the tuning's defaults, apply tiles of 64 columns by 8 rows (members need not be
+  // multiples of a wide tile) by a common number of planes kp, chosen as for one domain: the
+  // compute unit with most tiles ends the launch, n tiles of kp planes take n (kp + 1) plane
+  // times, and below `busy` tiles a unit idles.  Against whole columns of 256 by 2 tiles,
+  // solves of all members, us before / after: 7 members of 61 to 89 squared, 2x2, 3030/2253;
+  // 4 of 56 to 121, one component, 2274/1256; 7 of 51 to 159, 2x2, 4151/2982; 8 of 64 to
+  // 256, 2x2, 9379/9010.
+  const bool balance =
+      c->tune.apply_bx == 256 && c->tune.apply_zsplit == 1 && c->tune.apply_rows == 2;
+  const int bx = c->abx = balance ? 64 : c->tune.apply_bx;
   const int by = (256 / bx) * (c->tune.apply_rows == 2 ? 2 : 1);  // rows per apply tile
+  int kp = 0;
+  if (balance) {
+    const long busy = c->np1 == 1 ? 3 : 2;
+    double least = 0;
+    for (int k = 1; k <= c->maxnz; ++k) {
+      long tiles = 0;
+      for (const asam_sound_grid& q : c->grids)
+        tiles += (long)((q.nx + bx - 1) / bx) * ((q.ny + by - 1) / by) * ((q.nz + k - 1) / k);
+      const double cost = (double)std::max((tiles + c->ncu - 1) / c->ncu, busy) * (k + 1);
+      if (k == 1 || cost < least) {
+        least = cost;
+        kp = k;
+      }
+    }
+  }
   long gA = 0, gL = 0, gB = 0;
   for (int m = 0; m < c->nmem; ++m) {
     EnsMember& M = c->mh[m];
     M.agx = (M.nx + bx - 1) / bx;
     M.agy = (M.ny + by - 1) / by;
     const int zs = std::min(c->tune.apply_zsplit, M.nz);
-    M.akp = (M.nz + zs - 1) / zs;
+    M.akp = balance ? std::min(kp, M.nz) : (M.nz + zs - 1) / zs;
     const int nzt = (M.nz + M.akp - 1) / M.akp;
     const long ant = (long)M.agx * M.agy * nzt;
     M.lgx = (M.nx + 63) / 64;
@@ -543,11 +569,11 @@ static void ens_apply_go(asam_ens_ctx* c, dim3 grid, dim3 blk,
 template <int NP>
 void apply_outer(asam_ens_ctx* c, bool first, double* x, const double* b) {
   KEnsApply<double, double, float, float> e;
-  e.c = c->c64; e.mem = c->md; e.tmem = c->tA; e.ntiles = c->nA; e.bxw = c->tune.apply_bx;
+  e.c = c->c64; e.mem = c->md; e.tmem = c->tA; e.ntiles = c->nA; e.bxw = c->abx;
   e.xa = x; e.xb = c->xb; e.dx = c->d; e.b = b; e.y = c->r; e.y2 = c->rt; e.u = nullptr;
   e.partial = c->partial; e.pstride = c->pstride; e.st = c->st; e.skip_outer = 1;
   const dim3 grid(grid_for(c->nA, c->tune.apply_pf, c->ncu));
-  const dim3 blk(c->tune.apply_bx, 256 / c->tune.apply_bx);
+  const dim3 blk(c->abx, 256 / c->abx);
   if (first) {
     // a scan of the initial guess picks on the device which launch writes the residual:
     // the full FP64 apply, or for an all-zero guess the x = 0 form (b outside the dead
@@ -566,11 +592,11 @@ void apply_outer(asam_ens_ctx* c, bool first, double* x, const double* b) {
 template <int NP, int FL>
 void apply_inner(asam_ens_ctx* c, float* x, float* y, const float* u) {
   KEnsApply<float, float, float, float> e;
-  e.c = c->c32; e.mem = c->md; e.tmem = c->tA; e.ntiles = c->nA; e.bxw = c->tune.apply_bx;
+  e.c = c->c32; e.mem = c->md; e.tmem = c->tA; e.ntiles = c->nA; e.bxw = c->abx;
   e.xa = x; e.xb = nullptr; e.dx = nullptr; e.b = nullptr; e.y = y; e.y2 = nullptr; e.u = u;
   e.partial = c->partial; e.pstride = c->pstride; e.st = c->st; e.skip_outer = 0;
   ens_apply_go<NP, FL, 0>(c, dim3(grid_for(c->nA, c->tune.apply_pf, c->ncu)),
-                         dim3(c->tune.apply_bx, 256 / c->tune.apply_bx), e);
+                         dim3(c->abx, 256 / c->abx), e);
 }
 
 template <int NP, int MODE, int LDS, int P>

@@ -32,7 +32,8 @@ typedef struct asam_ens_ctx asam_ens_ctx;
 /* Launch shapes of the batched kernels (chosen by asam_ens_autotune). */
 typedef struct {
   int apply_bx;      /* stencil-apply tile width along x: 64, 128 or 256 (256 threads) */
-  int apply_zsplit;  /* tiles per column along z (1..8): each member's nz split evenly */
+  int apply_zsplit;  /* tiles per column along z (1..8): each member's nz split evenly.  At
+                        the defaults (256, 1, two rows) the tiles follow the members */
   int apply_pf;      /* workgroups per CU of the persistent apply grid; 0: one per tile */
   int line_window;   /* levels per load window of the line solve: 4 or 8 */
   int line_lds;      /* LDS budget of the line solve's forward sweep per workgroup: 0 none

@@ -96,8 +96,11 @@ typedef struct {
                         of rows plane by plane), 3: z-march of apply_rows rows of a column
                         per thread (the inner rows' y-neighbours come from registers) */
   int apply_wg;      /* target workgroups per stencil-apply launch (256..16384; variant 2:
-                        the workgroups of the launch, each looping over its XCD's tiles) */
-  int line_window;   /* levels per load window of the line solve: 1, 4 or 8 */
+                        the workgroups of the launch, each looping over its XCD's tiles).
+                        At the defaults of the apply_ fields the tile and the number of
+                        workgroups follow the grid */
+  int line_window;   /* levels per load window of the line solve: 1, 4 or 8; 0 (default):
+                        by the size of the grid */
   int line_lds;      /* LDS budget per workgroup for the line solve's forward sweep: 0 none
                         (staged in the output vector), 1 default (60 KiB), 2..160 that
                         many KiB; the lowest levels that fit are staged in LDS, the rest
@@ -117,9 +120,9 @@ typedef struct {
   int apply_band_rows; /* variant 2: rows per band (0: ny/8, one band per XCD) */
   int apply_rows;    /* variant 3: rows of a column each thread walks together, 2 or 4 */
   int line_nt;       /* cache policy of the line solve's factor loads (and of the vectors it
-                        reads once): 0 plain, 1 nontemporal, 2 (default) nontemporal when the
-                        factors of the solve's precision exceed 64 MiB, plain below, where
-                        they stay resident in the Infinity Cache.  Same bits either way */
+                        reads once): 0 plain, 1 nontemporal, 2 (default) nontemporal for
+                        factors too large to stay resident in the Infinity Cache between
+                        solves, plain below.  Same bits either way */
   int apply_depth;   /* variant 3 with FP32 coefficients, 2x2 blocks and two rows: the
                         levels a thread loads ahead of the one it computes, 1 (default;
                         the z-face coefficients and volumes then come from a packed copy,
