@@ -235,47 +235,110 @@ __global__ __launch_bounds__(256) void k_skew_fall(Dims d, const double* __restr
           wf[slot_row(d, jt, h, k) * (2 * kRow) + 2 * jj + q] = v;
         });
 }
-// Grid z: levels x groups x NC.
+// A vector to the skewed layout, the NC components of a group together (they lie side by side
+// there), kVecH rows h per block: half a wavefront loads a run of kVecH cells along x of one
+// column, the loads of all columns in flight together, and a wavefront stores a row.  Bound by
+// memory.  With one component per block the loads and stores of the skewed side move half of
+// each 16 bytes: 4 components of 256x256x64 took 120 us (k_skew_vec) and 189 us (k_unskew),
+// now 54 us and 56 us (4.9 TB/s).
+// Grid (y-tiles x runs of kVecH rows, 1, levels x groups).
+constexpr int kVecH = 32;
+constexpr int kMaxCols = 53;  // columns of a y-tile at most, see kMaxSweeps below
 template <int NC>
 __global__ __launch_bounds__(256) void k_skew_vec(Dims d, Groups gr, const double* __restrict__ v,
                                                   double* __restrict__ vs) {
-  __shared__ double t[64][kTileH + 1];
-  const int nh = h_blocks(d), jt = blockIdx.x / nh, h0 = (blockIdx.x - jt * nh) * kTileH;
-  const int e = blockIdx.z / d.Z, k = blockIdx.z - e * d.Z, g = e / NC, h = e - g * NC;
-  const double* const src = v + (long)gr.c[g][h] * d.m;
-  double* const dst = vs + g * d.slots * NC + h;
-  skew_tile(
-      d, jt, h0, t,
-      [&](int jj, int i) { return src[i + (long)d.X * (jt * d.TW + jj + (long)d.Y * k)]; },
-      [&](int h, int jj, double x) { dst[(slot_row(d, jt, h, k) * kRow + jj) * NC] = x; });
+  __shared__ double t[NC][kMaxCols][kVecH + 1];
+  const int nh = (d.HL + kVecH - 1) / kVecH, jt = blockIdx.x / nh, h0 = (blockIdx.x - jt * nh) * kVecH;
+  const int g = blockIdx.z / d.Z, k = blockIdx.z - g * d.Z;
+  const int rows = min(d.TW, d.Y - jt * d.TW);
+  {
+    const int l = threadIdx.x & (kVecH - 1), r0 = threadIdx.x / kVecH;
+    constexpr int RP = 256 / kVecH, NR = (kMaxCols + RP - 1) / RP;
+    double x[NR][NC];
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+      const int jj = r0 + q * RP, i = h0 + l - jj;
+      const bool in = jj < rows && i >= 0 && i < d.X;
+      const long cell = i + (long)d.X * (jt * d.TW + jj + (long)d.Y * k);
+#pragma unroll
+      for (int n = 0; n < NC; ++n) x[q][n] = in ? v[(long)gr.c[g][n] * d.m + cell] : 0.0;
+    }
+#pragma unroll
+    for (int q = 0; q < NR; ++q) {
+      const int jj = r0 + q * RP;
+      if (jj < rows) {
+#pragma unroll
+        for (int n = 0; n < NC; ++n) t[n][jj][l] = x[q][n];
+      }
+    }
+  }
+  __syncthreads();
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  double* const dst = vs + g * d.slots * NC;
+  for (int hh = wv; hh < kVecH; hh += 4) {
+    const int h = h0 + hh, i = h - lane;
+    if (lane < rows && h < d.HL && i >= 0 && i < d.X) {
+      double* const p = dst + (slot_row(d, jt, h, k) * kRow + lane) * NC;
+      if constexpr (NC == 2)
+        *reinterpret_cast<double2*>(p) = make_double2(t[0][lane][hh], t[1][lane][hh]);
+      else
+        *p = t[0][lane][hh];
+    }
+  }
 }
-// Back to the natural layout with the six halo faces zero (PSolveSp :734-739).  Grid
-// (y-tiles x runs of 64 cells along x, 1, levels x groups x NC).
+// Back to the natural layout with the six halo faces zero (PSolveSp :734-739), kVecH cells
+// along x of every column per block.  Grid (y-tiles x runs of kVecH cells along x, 1, levels x
+// groups).
 template <int NC>
 __global__ __launch_bounds__(256) void k_unskew(Dims d, Groups gr, const double* __restrict__ vs,
                                                 double* __restrict__ v) {
-  __shared__ double t[2 * kTileH][64 + 1];
-  const int nx = (d.X + kTileH - 1) / kTileH, jt = blockIdx.x / nx;
-  const int i0 = (blockIdx.x - jt * nx) * kTileH;
-  const int e = blockIdx.z / d.Z, k = blockIdx.z - e * d.Z, g = e / NC, n = e - g * NC;
-  const int c = gr.c[g][n];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  // cell i0 + l of column jj at 34 jj + l: a wavefront writes 33 jj + const, its own bank each
+  __shared__ double t[NC][kMaxCols][kVecH + 2];
+  const int nx = (d.X + kVecH - 1) / kVecH, jt = blockIdx.x / nx;
+  const int i0 = (blockIdx.x - jt * nx) * kVecH;
+  const int g = blockIdx.z / d.Z, k = blockIdx.z - g * d.Z;
   const int rows = min(d.TW, d.Y - jt * d.TW);
-  const double* src = vs + g * d.slots * NC + n;
   const bool inner_k = k >= 1 && k <= d.nz;
-  if (inner_k)
-    for (int hh = wv; hh < kTileH + d.TW - 1; hh += 4) {
-      const int h = i0 + hh, i = h - lane;
-      if (lane < rows && h < d.HL && i >= i0 && i < d.X)
-        t[hh][lane] = src[(slot_row(d, jt, h, k) * kRow + lane) * NC];
+  if (inner_k) {
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const double* src = vs + g * d.slots * NC;
+    constexpr int NH = (kVecH + kMaxCols - 1 + 3) / 4;  // rows h of a wavefront
+    double x[NH][NC];
+#pragma unroll
+    for (int q = 0; q < NH; ++q) {
+      const int l = wv + 4 * q - lane, h = i0 + wv + 4 * q;
+      const bool in = lane < rows && l >= 0 && l < kVecH && i0 + l < d.X;
+      const double* const p = src + (slot_row(d, jt, h, k) * kRow + lane) * NC;
+#pragma unroll
+      for (int n = 0; n < NC; ++n) x[q][n] = 0.0;
+      if (in) {
+        if constexpr (NC == 2) {
+          const double2 w = *reinterpret_cast<const double2*>(p);
+          x[q][0] = w.x;
+          x[q][1] = w.y;
+        } else {
+          x[q][0] = *p;
+        }
+      }
     }
+#pragma unroll
+    for (int q = 0; q < NH; ++q) {
+      const int l = wv + 4 * q - lane;
+      if (lane < rows && l >= 0 && l < kVecH) {
+#pragma unroll
+        for (int n = 0; n < NC; ++n) t[n][lane][l] = x[q][n];
+      }
+    }
+  }
   __syncthreads();
-  const int i = i0 + lane;
+  const int l = threadIdx.x & (kVecH - 1), i = i0 + l;
   if (i >= d.X) return;
-  for (int jj = wv; jj < rows; jj += 4) {
+  for (int jj = threadIdx.x / kVecH; jj < rows; jj += 256 / kVecH) {
     const int j = jt * d.TW + jj;
     const bool in = inner_k && i >= 1 && i <= d.nx && j >= 1 && j <= d.ny;
-    v[(long)c * d.m + i + (long)d.X * (j + (long)d.Y * k)] = in ? t[lane + jj][jj] : 0.0;
+#pragma unroll
+    for (int n = 0; n < NC; ++n)
+      v[(long)gr.c[g][n] * d.m + i + (long)d.X * (j + (long)d.Y * k)] = in ? t[n][jj][l] : 0.0;
   }
 }
 
@@ -288,9 +351,8 @@ __global__ void k_zero_int(int* p, int n) {
 // Sweeps one launch runs at most: six wavefronts, the polling and the storing one; two such
 // blocks fit a CU.
 constexpr int kMaxSweeps = 6;
-// Columns of a y-tile at most: a step's values of the top level of a block are five runs of 64
-// (64 columns would take six, and the spare lanes cost less than the extra polls).
-constexpr int kMaxCols = 53;
+// Columns of a y-tile at most (kMaxCols): a step's values of the top level of a block are five
+// runs of 64 (64 columns would take six, and the spare lanes cost less than the extra polls).
 constexpr unsigned long long kSentinel = 0xFFF7DEADBEEF0001ull;  // NaN payload: not yet
 
 struct GsArgs {
@@ -1231,13 +1293,14 @@ template <int NC>
 static int psolve_nc(asam_tr_ctx* c, const double* x, double* y) {
   const Dims& d = c->d;
   const Groups gr = make_groups(c, NC);
-  const int levels = d.Z * gr.n * NC;
+  const int levels = d.Z * gr.n;
   k_zero_int<<<1, 64, 0, c->stream>>>(c->sync + 1, 1);
-  k_skew_vec<NC><<<skew_grid(d, levels), 256, 0, c->stream>>>(d, gr, x, c->bs);
+  k_skew_vec<NC><<<dim3(d.NJ * ((d.HL + kVecH - 1) / kVecH), 1, levels), 256, 0, c->stream>>>(
+      d, gr, x, c->bs);
   TRCHK(c, hipGetLastError());
   for (size_t q = 0; q < c->groups.size(); ++q)
     if (int rc = launch_sweeps<NC>(c, gr, c->groups[q], q == 0)) return rc;
-  k_unskew<NC><<<dim3(d.NJ * ((d.X + kTileH - 1) / kTileH), 1, levels), 256, 0, c->stream>>>(
+  k_unskew<NC><<<dim3(d.NJ * ((d.X + kVecH - 1) / kVecH), 1, levels), 256, 0, c->stream>>>(
       d, gr, c->xs, y);
   TRCHK(c, hipGetLastError());
   return 0;
