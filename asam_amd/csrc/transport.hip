@@ -34,7 +34,6 @@ namespace asam {
 namespace tr {
 
 constexpr int kMaxComp = ASAM_TR_MAX_COMP;
-constexpr int kDotBlocks = 1024;
 constexpr int kSpinLimit = 1 << 22;
 
 struct Ops {
@@ -57,17 +56,27 @@ struct Groups {
 };
 
 __device__ __forceinline__ bool is_interior(const Dims& d, long r, int& i, int& j, int& k) {
-  i = (int)(r % d.X);
-  const long t = r / d.X;
-  j = (int)(t % d.Y);
-  k = (int)(t / d.Y);
+  if (d.m <= 0xffffffffl) {  // uniform; 32-bit divisions take a quarter of the instructions
+    const unsigned u = (unsigned)r, w = u / (unsigned)d.X, z = w / (unsigned)d.Y;
+    i = (int)(u - w * (unsigned)d.X);
+    j = (int)(w - z * (unsigned)d.Y);
+    k = (int)z;
+  } else {
+    i = (int)(r % d.X);
+    const long w = r / d.X;
+    j = (int)(w % d.Y);
+    k = (int)(w / d.Y);
+  }
   return i >= 1 && i <= d.nx && j >= 1 && j <= d.ny && k >= 1 && k <= d.nz;
 }
 
 // ------------------------------------------------------------------ operator (MatVec)
 // y = x + LU^-1 (T x - x) on interior cells, T x on the halo, for all components at once
 // (MatVecChem/Met_Vec4CellSp: SpAVec, Axpy(-1), PSolveMatrix, Xpy).  The 7 (14 with
-// JacTMom) coefficients of a cell are read once for every component.
+// JacTMom) coefficients of a cell are read once for every component.  Over the interior cells
+// also the sums of y u (nd >= 1) and y y (nd = 2), one partial sum per block: for 4 reacting
+// components of 256x256x64 that adds 20 us to the 262 us of the launch, where the dots by
+// themselves took 69 us and 82 us.
 template <int NC>
 __global__ __launch_bounds__(256) void k_matvec(Dims d, const double* __restrict__ tmom,
                                                 const double* __restrict__ tpot,
@@ -75,10 +84,14 @@ __global__ __launch_bounds__(256) void k_matvec(Dims d, const double* __restrict
                                                 const double* __restrict__ lu,
                                                 const double* __restrict__ x,
                                                 double* __restrict__ y, Ops ops, int init,
-                                                int use_mom, int use_pot) {
+                                                int use_mom, int use_pot, int nd,
+                                                const double* __restrict__ u,
+                                                double* __restrict__ partial) {
 #pragma clang fp contract(off)
-  const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= d.m) return;
+  const long r0 = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  const bool live = r0 < d.m;
+  if (!live && nd == 0) return;
+  const long r = live ? r0 : d.m - 1;
   const long XY = (long)d.X * d.Y;
   const long off[7] = {-XY, -(long)d.X, -1, 0, 1, (long)d.X, XY};
   double vp[7], vm[7];
@@ -107,8 +120,9 @@ __global__ __launch_bounds__(256) void k_matvec(Dims d, const double* __restrict
     }
     s[c] = -1.0 * xc[r] + acc;
   }
-  int i, j, k;
-  if (lu && is_interior(d, r, i, j, k)) {
+  int i = 0, j = 0, k = 0;
+  const bool in = (lu || nd > 0) && is_interior(d, r, i, j, k);
+  if (lu && in) {
     const long q = (i - 1) + (long)d.nx * ((j - 1) + (long)d.ny * (k - 1));
 #pragma unroll
     for (int kc = 0; kc < NC; ++kc)
@@ -123,8 +137,17 @@ __global__ __launch_bounds__(256) void k_matvec(Dims d, const double* __restrict
         s[ic] = s[ic] - lu[((long)ic * NC + kc) * d.ncell + q] * s[kc];
     }
   }
+  double acc[2] = {0.0, 0.0};
 #pragma unroll
-  for (int c = 0; c < NC; ++c) y[c * d.m + r] = x[c * d.m + r] + s[c];
+  for (int c = 0; c < NC; ++c) {
+    const double yc = x[c * d.m + r] + s[c];
+    if (live) y[c * d.m + r] = yc;
+    if (nd > 0 && live && in) {
+      acc[0] = __builtin_fma(yc, u[c * d.m + r], acc[0]);
+      acc[1] = __builtin_fma(yc, yc, acc[1]);
+    }
+  }
+  if (nd > 0) block_reduce_store<2>(acc, partial, blockIdx.x, threadIdx.x, 256, gridDim.x);
 }
 
 // ------------------------------------------------------------------ division
@@ -792,41 +815,109 @@ __global__ __launch_bounds__(512, 2) void k_gs_tiles(GsArgs a, Ops ops) {
 }
 
 // ------------------------------------------------------------------ dots and updates
-// Sums over the interior cells of all components of NQ products a_q . b_q.
-template <int NQ>
-__global__ __launch_bounds__(256) void k_dot(Dims d, int nc, const double* __restrict__ a0,
-                                             const double* __restrict__ b0,
-                                             const double* __restrict__ a1,
-                                             const double* __restrict__ b1,
-                                             double* __restrict__ partial) {
-  double acc[NQ];
+// The vector steps of the solve, each one pass over its vectors with the sums that follow it
+// (over the interior cells, one partial sum per block).  Bound by memory; 4 components of
+// 256x256x64 (138 MB a vector): the last step of an iteration moves 8 vectors in 198 us,
+// where three updates and two dots took 330 us for 12.
+constexpr int kStepElems = 4;  // elements of a thread
+template <typename F>
+__device__ __forceinline__ void step_elems(const Dims& d, int nc, F&& f) {
+  const long n = (long)nc * d.m;
+  const long e0 = (long)blockIdx.x * (256 * kStepElems) + threadIdx.x;
 #pragma unroll
-  for (int q = 0; q < NQ; ++q) acc[q] = 0.0;
-  const long total = (long)nc * d.ncell;
-  for (long e = (long)blockIdx.x * blockDim.x + threadIdx.x; e < total;
-       e += (long)gridDim.x * blockDim.x) {
-    const long c = e / d.ncell, q = e - c * d.ncell;
-    const long i = q % d.nx, t = q / d.nx;
-    const long jj = t % d.ny, k = t / d.ny;
-    const long r = c * d.m + (i + 1) + d.X * ((jj + 1) + (long)d.Y * (k + 1));
-    acc[0] += a0[r] * b0[r];
-    if (NQ > 1) acc[NQ - 1] += a1[r] * b1[r];
+  for (int q = 0; q < kStepElems; ++q) {
+    const long e = e0 + q * 256;
+    if (e >= n) break;
+    long r = e;
+    if (nc > 1) r -= d.m * (n <= 0xffffffffl ? (long)((unsigned)e / (unsigned)d.m) : e / d.m);
+    int i, j, k;
+    f(e, is_interior(d, r, i, j, k));
   }
-  block_reduce_store<NQ>(acc, partial, blockIdx.x, threadIdx.x, blockDim.x, kDotBlocks);
 }
-// Fixed-order sum of the partials: thread t adds partials t, t+1024, ... (one each here),
-// then the block tree; every run gives the same bits.
-template <int NQ>
+// r = b - r (r = A x on entry); rt = p = r; r.r.
+__global__ __launch_bounds__(256) void k_step_init(Dims d, int nc, const double* __restrict__ b,
+                                                   double* __restrict__ r,
+                                                   double* __restrict__ rt,
+                                                   double* __restrict__ p,
+                                                   double* __restrict__ partial) {
+#pragma clang fp contract(off)
+  double acc[2] = {0.0, 0.0};
+  step_elems(d, nc, [&](long e, bool in) {
+    const double v = -1.0 * r[e] + b[e];
+    r[e] = v;
+    rt[e] = v;
+    p[e] = v;
+    if (in) acc[0] = __builtin_fma(v, v, acc[0]);
+  });
+  block_reduce_store<2>(acc, partial, blockIdx.x, threadIdx.x, 256, gridDim.x);
+}
+// p = r + beta (p - omega v); an update by zero is left out (Axpy_VectorCell :1243).
+__global__ __launch_bounds__(256) void k_step_dir(long n, double omega, double beta,
+                                                  const double* __restrict__ v,
+                                                  const double* __restrict__ r,
+                                                  double* __restrict__ p) {
+#pragma clang fp contract(off)
+  const long e = (long)blockIdx.x * 256 + threadIdx.x;
+  if (e >= n) return;
+  double q = p[e];
+  if (omega != 0.0) q = -omega * v[e] + q;
+  p[e] = beta * q + r[e];
+}
+// s = r - alpha v (into r); s.s.
+__global__ __launch_bounds__(256) void k_step_half(Dims d, int nc, double alpha,
+                                                   const double* __restrict__ v,
+                                                   double* __restrict__ r,
+                                                   double* __restrict__ partial) {
+#pragma clang fp contract(off)
+  double acc[2] = {0.0, 0.0};
+  step_elems(d, nc, [&](long e, bool in) {
+    double s = r[e];
+    if (alpha != 0.0) {
+      s = -alpha * v[e] + s;
+      r[e] = s;
+    }
+    if (in) acc[0] = __builtin_fma(s, s, acc[0]);
+  });
+  block_reduce_store<2>(acc, partial, blockIdx.x, threadIdx.x, 256, gridDim.x);
+}
+// x += alpha ph + omega rh; r = s - omega t; r.r and rt.r (the next iteration's rho).
+__global__ __launch_bounds__(256) void k_step_full(Dims d, int nc, double alpha, double omega,
+                                                   const double* __restrict__ ph,
+                                                   const double* __restrict__ rh,
+                                                   const double* __restrict__ t,
+                                                   const double* __restrict__ rt,
+                                                   double* __restrict__ x,
+                                                   double* __restrict__ r,
+                                                   double* __restrict__ partial) {
+#pragma clang fp contract(off)
+  double acc[2] = {0.0, 0.0};
+  step_elems(d, nc, [&](long e, bool in) {
+    double xe = x[e], re = r[e];
+    if (alpha != 0.0) xe = alpha * ph[e] + xe;
+    if (omega != 0.0) {
+      xe = omega * rh[e] + xe;
+      re = -omega * t[e] + re;
+    }
+    x[e] = xe;
+    r[e] = re;
+    if (in) {
+      acc[0] = __builtin_fma(re, re, acc[0]);
+      acc[1] = __builtin_fma(rt[e], re, acc[1]);
+    }
+  });
+  block_reduce_store<2>(acc, partial, blockIdx.x, threadIdx.x, 256, gridDim.x);
+}
+// Fixed-order sums of the two partial sums of nblk blocks: thread t adds partials t, t + 1024,
+// ..., then the block tree; every run gives the same bits.
 __global__ __launch_bounds__(1024) void k_dot_fin(const double* __restrict__ partial, int nblk,
                                                   double* __restrict__ out) {
-  double v[NQ];
-#pragma unroll
-  for (int q = 0; q < NQ; ++q) {
-    double s = 0.0;
-    for (int b = threadIdx.x; b < nblk; b += blockDim.x) s += partial[q * kDotBlocks + b];
-    v[q] = s;
+  double v[2] = {0.0, 0.0};
+#pragma unroll 4
+  for (int b = threadIdx.x; b < nblk; b += 1024) {
+    v[0] += partial[b];
+    v[1] += partial[nblk + b];
   }
-  block_reduce_store<NQ>(v, out, 0, threadIdx.x, blockDim.x, 1);
+  block_reduce_store<2>(v, out, 0, threadIdx.x, 1024, 1);
 }
 
 __global__ void k_axpy(long n, double a, const double* __restrict__ x, double* __restrict__ y) {
@@ -834,12 +925,6 @@ __global__ void k_axpy(long n, double a, const double* __restrict__ x, double* _
   const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (e < n) y[e] = a * x[e] + y[e];
 }
-__global__ void k_xpay(long n, const double* __restrict__ x, double a, double* __restrict__ y) {
-#pragma clang fp contract(off)
-  const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < n) y[e] = a * y[e] + x[e];
-}
-
 }  // namespace tr
 }  // namespace asam
 
@@ -902,6 +987,9 @@ static int tralloc(asam_tr_ctx* c, T** p, size_t count) {
 }
 
 static inline unsigned blocks_for(long n, int bs) { return (unsigned)((n + bs - 1) / bs); }
+static inline long step_blocks(const asam_tr_ctx* c) {
+  return blocks_for((long)c->nc * c->d.m, 256 * kStepElems);
+}
 
 // Rows of a skewed array in front and behind that lanes without a cell may read.
 constexpr int kGuardRows = 16;
@@ -994,7 +1082,7 @@ extern "C" int asam_tr_create(asam_tr_ctx** out, const asam_tr_grid* g) {
   double** vecs[] = {&c->vx, &c->vb, &c->vr, &c->vrt, &c->vrh, &c->vp, &c->vph, &c->vt, &c->vv,
                      &c->vh};
   for (double** v : vecs) rc |= tralloc(c, v, V);
-  rc |= tralloc(c, &c->partial, 2 * (size_t)kDotBlocks);
+  rc |= tralloc(c, &c->partial, 2 * (size_t)std::max((long)blocks_for(d.m, 256), step_blocks(c)));
   rc |= tralloc(c, &c->dots, 2);
   c->sync_n = 3;  // ticket, error word, set-up flag
   rc |= tralloc(c, &c->sync, (size_t)c->sync_n);
@@ -1113,19 +1201,22 @@ static int check_ready(asam_tr_ctx* c, const Ops& o) {
 }
 
 template <int NC>
-static void matvec_nc(asam_tr_ctx* c, const double* x, double* y, int init, int mom) {
+static void matvec_nc(asam_tr_ctx* c, const double* x, double* y, int init, int mom, int nd,
+                      const double* u) {
   const Dims& d = c->d;
   k_matvec<NC><<<blocks_for(d.m, 256), 256, 0, c->stream>>>(
       d, c->tmom, c->tpot, c->fall, c->have_lu ? c->lu : nullptr, x, y, c->ops_mv, init, mom,
-      1);
+      1, nd, u, c->partial);
 }
 
-static int launch_matvec(asam_tr_ctx* c, const double* x, double* y, int init) {
+// nd sums over the interior cells with it: y.u (1), y.y (2), see sums().
+static int launch_matvec(asam_tr_ctx* c, const double* x, double* y, int init, int nd = 0,
+                         const double* u = nullptr) {
   const int mom = (!init && uses(c->ops_mv, c->nc, ASAM_TR_MOM)) ? 1 : 0;
   switch (c->nc) {
 #define NCCASE(n) \
   case n:         \
-    matvec_nc<n>(c, x, y, init, mom); \
+    matvec_nc<n>(c, x, y, init, mom, nd, u); \
     break;
     NCCASE(1) NCCASE(2) NCCASE(3) NCCASE(4) NCCASE(5) NCCASE(6) NCCASE(7) NCCASE(8)
     NCCASE(9) NCCASE(10) NCCASE(11) NCCASE(12) NCCASE(13) NCCASE(14) NCCASE(15) NCCASE(16)
@@ -1320,17 +1411,15 @@ static int check_gs_error(asam_tr_ctx* c) {
   return 0;
 }
 
-// NQ dots over the interior cells; results on the host.
-template <int NQ>
-static int dots(asam_tr_ctx* c, const double* a0, const double* b0, const double* a1,
-                const double* b1, double* out) {
-  k_dot<NQ><<<kDotBlocks, 256, 0, c->stream>>>(c->d, c->nc, a0, b0, a1, b1, c->partial);
-  k_dot_fin<NQ><<<1, 1024, 0, c->stream>>>(c->partial, kDotBlocks, c->dots);
+// The two sums of the nblk blocks launched last; results on the host.
+static int sums(asam_tr_ctx* c, long nblk, double* out) {
+  k_dot_fin<<<1, 1024, 0, c->stream>>>(c->partial, (int)nblk, c->dots);
   TRCHK(c, hipGetLastError());
-  TRCHK(c, hipMemcpyAsync(c->host_dots, c->dots, NQ * sizeof(double), hipMemcpyDeviceToHost,
+  TRCHK(c, hipMemcpyAsync(c->host_dots, c->dots, 2 * sizeof(double), hipMemcpyDeviceToHost,
                           c->stream));
   TRCHK(c, hipStreamSynchronize(c->stream));
-  for (int q = 0; q < NQ; ++q) out[q] = c->host_dots[q];
+  out[0] = c->host_dots[0];
+  out[1] = c->host_dots[1];
   return 0;
 }
 
@@ -1341,18 +1430,6 @@ static int axpy(asam_tr_ctx* c, double a, const double* x, double* y) {
   TRCHK(c, hipGetLastError());
   return 0;
 }
-static int xpay(asam_tr_ctx* c, const double* x, double a, double* y) {
-  const long V = (long)c->nc * c->d.m;
-  k_xpay<<<blocks_for(V, 256), 256, 0, c->stream>>>(V, x, a, y);
-  TRCHK(c, hipGetLastError());
-  return 0;
-}
-static int copy(asam_tr_ctx* c, const double* x, double* y) {
-  TRCHK(c, hipMemcpyAsync(y, x, sizeof(double) * c->nc * c->d.m, hipMemcpyDeviceToDevice,
-                          c->stream));
-  return 0;
-}
-
 #define TRY(expr)              \
   do {                         \
     if (int rc_ = (expr)) return rc_; \
@@ -1368,40 +1445,37 @@ static int solve_dev(asam_tr_ctx* c, double* x, const double* b, int* maxiter, d
   const double Tol = *tol;
   TRY(launch_matvec(c, x, r, 1));  // MatVecChem(r, A, x)
   inf.matvecs = 1;
-  TRY(xpay(c, b, -1.0, r));        // r = b - r
-  TRY(copy(c, r, rt));
+  const Dims& d = c->d;
+  const long V = (long)c->nc * d.m, sb = step_blocks(c), mb = blocks_for(d.m, 256);
   double q2[2];
-  TRY(dots<1>(c, r, r, nullptr, nullptr, q2));
+  k_step_init<<<(unsigned)sb, 256, 0, c->stream>>>(d, c->nc, b, r, rt, p, c->partial);
+  TRY(sums(c, sb, q2));
   const double rnorm0 = std::sqrt(q2[0]);
   inf.rnorm0 = rnorm0;
   inf.rnorm = rnorm0;
   inf.status = ASAM_NOT_CONVERGED;
-  double rho = 0.0, rho_old, alpha = 0.0, omega = 0.0, beta, rnorm = rnorm0;
+  double rho = 0.0, rho_old, rho_next = q2[0], alpha = 0.0, omega = 0.0, beta, rnorm = rnorm0;
   for (int it = 1; it <= MaxIter; ++it) {
     inf.iterations = it;
     rho_old = rho;
-    TRY(dots<1>(c, rt, r, nullptr, nullptr, q2));
-    rho = q2[0];
+    rho = rho_next;  // rt.r, with the step that wrote r (rt = r at first)
     if (rho == 0.0) {
       *maxiter = it;
       *tol = 0.0;
       inf.status = ASAM_BREAKDOWN;
       break;
     }
-    if (it == 1) {
-      TRY(copy(c, r, p));
-    } else {
+    if (it > 1) {  // p = r at first
       beta = (rho / rho_old) * (alpha / omega);
-      TRY(axpy(c, -omega, v, p));
-      TRY(xpay(c, r, beta, p));
+      k_step_dir<<<blocks_for(V, 256), 256, 0, c->stream>>>(V, omega, beta, v, r, p);
     }
     TRY(launch_psolve(c, p, ph));
-    TRY(launch_matvec(c, ph, v, 0));
+    TRY(launch_matvec(c, ph, v, 0, 1, rt));
     inf.psolves++, inf.matvecs++;
-    TRY(dots<1>(c, rt, v, nullptr, nullptr, q2));
+    TRY(sums(c, mb, q2));
     alpha = rho / q2[0];
-    TRY(axpy(c, -alpha, v, r));
-    TRY(dots<1>(c, r, r, nullptr, nullptr, q2));
+    k_step_half<<<(unsigned)sb, 256, 0, c->stream>>>(d, c->nc, alpha, v, r, c->partial);
+    TRY(sums(c, sb, q2));
     rnorm = std::sqrt(q2[0]);
     if (rnorm <= Tol * rnorm0) {
       TRY(axpy(c, alpha, ph, x));
@@ -1411,15 +1485,15 @@ static int solve_dev(asam_tr_ctx* c, double* x, const double* b, int* maxiter, d
       break;
     }
     TRY(launch_psolve(c, r, rh));
-    TRY(launch_matvec(c, rh, t, 0));
+    TRY(launch_matvec(c, rh, t, 0, 2, r));
     inf.psolves++, inf.matvecs++;
-    TRY(dots<2>(c, t, r, t, t, q2));
+    TRY(sums(c, mb, q2));
     omega = q2[0] / q2[1];
-    TRY(axpy(c, alpha, ph, x));
-    TRY(axpy(c, omega, rh, x));
-    TRY(axpy(c, -omega, t, r));
-    TRY(dots<1>(c, r, r, nullptr, nullptr, q2));
+    k_step_full<<<(unsigned)sb, 256, 0, c->stream>>>(d, c->nc, alpha, omega, ph, rh, t, rt, x, r,
+                                                     c->partial);
+    TRY(sums(c, sb, q2));
     rnorm = std::sqrt(q2[0]);
+    rho_next = q2[1];
     if (rnorm <= Tol * rnorm0) {
       *maxiter = it;
       *tol = rnorm;
