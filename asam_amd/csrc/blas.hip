@@ -5,6 +5,9 @@
 // then LDS across waves, one partial per workgroup); stage 2 is a
 // one-workgroup finalize kernel that sums the partials in a fixed order, so a
 // dot product is bitwise reproducible run to run.
+#include <algorithm>
+#include <type_traits>
+
 #include <math.h>
 #include <stdint.h>
 
@@ -90,22 +93,6 @@ void launch_bicg_update(hipStream_t s, long n, int vt, void* x, const void* ph, 
 }
 
 // ------------------------------------------------------------- (F)GMRES MGS
-// Sum of the nb partial products of the previous pass, in the same fixed order in every
-// workgroup (so every workgroup holds the same bits); all threads must take part.
-__device__ double block_sum_partials(const double* p, int nb) {
-  __shared__ double sh[4];
-  __shared__ double total;
-  const int tid = threadIdx.x;
-  double v = 0.0;
-  for (int b = tid; b < nb; b += 256) v += p[b];
-  v = wave_sum(v);
-  if ((tid & 63) == 0) sh[tid >> 6] = v;
-  __syncthreads();
-  if (tid == 0) total = (sh[0] + sh[1]) + (sh[2] + sh[3]);
-  __syncthreads();
-  return total;
-}
-
 // 16-byte packs of a vector: W = 4 floats or 2 doubles per load and store.  The FP32
 // passes of the Gram-Schmidt chains are latency-bound with one element per lane (half the
 // bytes in flight of the FP64 passes at the same speed), so the kernels below stream
@@ -143,124 +130,214 @@ __device__ __forceinline__ Pk<VT> zpk() {
 }
 __host__ inline bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
-// One element of a modified Gram-Schmidt pass: w -= h (v_prev * sp) (k > 0), rounded to
-// the vector type; then the product with v_k * sk, or w.w on the step's last pass.
-template <typename VT>
-__device__ __forceinline__ VT mgs_elem(VT w, VT vp, VT vk, int k, bool self, double h,
-                                       double sp, double sk, double& acc) {
-  double wv = (double)w;
-  if (k > 0) {
-    wv = wv + (-h) * ((double)vp * sp);
-    w = (VT)wv;
-    wv = (double)w;
-  }
-  if (self) acc += wv * wv;
-  else acc += ((double)vk * sk) * wv;
-  return w;
-}
-
-// hsrc: null, or the partial products of the previous pass of the chain; then H(k-1, i) is
-// their sum, formed here (workgroup 0 records it) instead of by a finalize launch.
-// PK: the vectors stream in 16-byte packs (every pointer aligned), the n mod W last
-// elements one per thread.
-template <typename VT, bool PK>
-__global__ __launch_bounds__(256) void k_mgs(long n, VT* __restrict__ w,
-                                             const VT* __restrict__ vprev,
-                                             const VT* __restrict__ vk, int k, int i,
-                                             KState* st, double* partial, int chk_done,
-                                             const double* hsrc, int hnb) {
+// w.w (NN = 0) or w.(v_0 vscale_0), where no stencil apply delivers it.
+template <typename VT, bool SELF>
+__global__ __launch_bounds__(256) void k_gm_dot(long n, const VT* __restrict__ w,
+                                                const VT* __restrict__ v0, const KState* st,
+                                                double* partial, int chk_done) {
   if (chk_done ? st->done : st->cycle_done) return;
-  double h = 0.0, sp = 0.0, sk = 0.0;
-  if (k > 0) {
-    if (hsrc) {
-      h = block_sum_partials(hsrc, hnb);
-      if (blockIdx.x == 0 && threadIdx.x == 0) st->H[(k - 1) * kMaxM + i] = h;
-    } else {
-      h = st->H[(k - 1) * kMaxM + i];
-    }
-    sp = st->vscale[k - 1];
-  }
-  const bool self = (k == i + 1);
-  if (!self) sk = st->vscale[k];
+  const double s0 = SELF ? 0.0 : st->vscale[0];
   double acc[1] = {0.0};
   const long stride = (long)gridDim.x * blockDim.x;
-  const long gid = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if constexpr (PK) {
-    constexpr int W = Pk<VT>::W, U = 2;
-    const long nc = n / W;
-    long c0 = gid;
-    // whole turns: U packs per thread, all loads first
-    for (; c0 + (U - 1) * stride < nc; c0 += U * stride) {
-      Pk<VT> wl[U], pl[U], kl[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const long c = c0 + u * stride;
-        wl[u] = ldpk(w, c);
-        pl[u] = k > 0 ? ldpk(vprev, c) : zpk<VT>();
-        kl[u] = !self ? ldpk(vk, c) : zpk<VT>();
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-#pragma unroll
-        for (int j = 0; j < W; ++j)
-          wl[u].v[j] = mgs_elem(wl[u].v[j], pl[u].v[j], kl[u].v[j], k, self, h, sp, sk, acc[0]);
-        if (k > 0) stpk(w, c0 + u * stride, wl[u]);
-      }
-    }
-    for (; c0 < nc; c0 += stride) {
-      Pk<VT> wl = ldpk(w, c0);
-      const Pk<VT> pl = k > 0 ? ldpk(vprev, c0) : zpk<VT>();
-      const Pk<VT> kl = !self ? ldpk(vk, c0) : zpk<VT>();
-#pragma unroll
-      for (int j = 0; j < W; ++j)
-        wl.v[j] = mgs_elem(wl.v[j], pl.v[j], kl.v[j], k, self, h, sp, sk, acc[0]);
-      if (k > 0) stpk(w, c0, wl);
-    }
-    const long e = nc * W + gid;
-    if (e < n) {
-      const VT r = mgs_elem(w[e], k > 0 ? vprev[e] : (VT)0, !self ? vk[e] : (VT)0, k, self, h,
-                            sp, sk, acc[0]);
-      if (k > 0) w[e] = r;
-    }
-  } else {
-    // U turns of the grid-stride loop at a time: the loads of all U elements first, then
-    // their arithmetic in the plain loop's order (same elements, same sums, same bits)
-    constexpr int U = 4;
-    for (long e0 = gid; e0 < n; e0 += U * stride) {
-      VT wl[U], pl[U], kl[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const long e = e0 + u * stride;
-        const bool ok = e < n;
-        wl[u] = ok ? w[e] : (VT)0;
-        pl[u] = (ok && k > 0) ? vprev[e] : (VT)0;
-        kl[u] = (ok && !self) ? vk[e] : (VT)0;
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const long e = e0 + u * stride;
-        if (e < n) {
-          const VT r = mgs_elem(wl[u], pl[u], kl[u], k, self, h, sp, sk, acc[0]);
-          if (k > 0) w[e] = r;
-        }
-      }
-    }
+#pragma unroll 4
+  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < n; e += stride) {
+    const double wv = (double)w[e];
+    acc[0] += SELF ? wv * wv : ((double)v0[e] * s0) * wv;
   }
   block_reduce_store_b<1>(acc, partial, blockIdx.x);
 }
 
-void launch_mgs(hipStream_t s, long n, int vt, void* w, const void* vprev, const void* vk, int k,
-                int i, KState* st, double* partial, int chk_done, const double* hsrc) {
+void launch_gm_dot(hipStream_t s, long n, int vt, const void* w, const void* v0, KState* st,
+                   double* partial, int chk_done) {
   const int nb = blas_blocks(n);
-  const bool pk = al16(w) && (k == 0 || al16(vprev)) && (!vk || al16(vk));
   if (vt == 0) {
-    auto f = pk ? k_mgs<double, true> : k_mgs<double, false>;
-    hipLaunchKernelGGL(f, dim3(nb), dim3(256), 0, s, n, (double*)w, (const double*)vprev,
-                       (const double*)vk, k, i, st, partial, chk_done, hsrc, nb);
+    auto f = v0 ? k_gm_dot<double, false> : k_gm_dot<double, true>;
+    hipLaunchKernelGGL(f, dim3(nb), dim3(256), 0, s, n, (const double*)w, (const double*)v0, st,
+                       partial, chk_done);
   } else {
-    auto f = pk ? k_mgs<float, true> : k_mgs<float, false>;
-    hipLaunchKernelGGL(f, dim3(nb), dim3(256), 0, s, n, (float*)w, (const float*)vprev,
-                       (const float*)vk, k, i, st, partial, chk_done, hsrc, nb);
+    auto f = v0 ? k_gm_dot<float, false> : k_gm_dot<float, true>;
+    hipLaunchKernelGGL(f, dim3(nb), dim3(256), 0, s, n, (const float*)w, (const float*)v0, st,
+                       partial, chk_done);
+  }
+}
+
+// One pass of the modified Gram-Schmidt of Arnoldi step i (SpMatrix4CellPar_Mod.f90 takes a
+// vector at a time): removes the projections on NP basis vectors k0 .. k0 + NP - 1 from w and
+// forms the products of the result with the NN vectors after them, or w.w when none is left
+// (NN = 0).  Taking kMgsBlock vectors at a time moves 2 + 2/kMgsBlock vectors per projection
+// instead of 4: FP64 256x256x64 one component, ten steps of a restart cycle, 55 launches of
+// 16.8 us (0.92 ms) before, 28 launches in 0.63 ms together now (7 to 10 TB/s).  The projections stay those of the
+// modified method: with d_a = v_a.w before the block and g_ab = v_a.v_b,
+//   h_a = d_a - sum over b < a of g_ab h_b,
+// where the g_ab, of rounding size, come from the same pass as the d_a.
+//
+// hsrc: null, or the partial sums of the pass before (NP products, then the g_ab); each
+// workgroup adds them up in the same order and the first one records the h_a in H.  The first
+// pass of a step has NP = 1 and takes h_0 from H.
+constexpr int kMgsSums = kMgsBlock + kMgsBlock * (kMgsBlock - 1) / 2;
+struct MgsVecs {
+  const void* prev[kMgsBlock];
+  const void* next[kMgsBlock];
+};
+template <typename VT, bool PK, int NP, int NN>
+__global__ __launch_bounds__(256) void k_mgs(long n, VT* __restrict__ w, MgsVecs vs, int k0,
+                                             int i, KState* st, double* partial,
+                                             const double* hsrc) {
+  if (st->cycle_done) return;
+  const int nb = gridDim.x, tid = threadIdx.x;
+  constexpr int NS = NP + NP * (NP - 1) / 2;              // sums this pass consumes
+  constexpr int NO = NN ? NN + NN * (NN - 1) / 2 : 1;     // and forms
+  double h[NP];
+  if (hsrc) {
+    __shared__ double sh[NS][4];
+    double v[NS];
+#pragma unroll
+    for (int q = 0; q < NS; ++q) {
+      v[q] = 0.0;
+      for (int b = tid; b < nb; b += 256) v[q] += hsrc[q * kMgsStride + b];
+    }
+#pragma unroll
+    for (int q = 0; q < NS; ++q) {
+      v[q] = wave_sum(v[q]);
+      if ((tid & 63) == 0) sh[q][tid >> 6] = v[q];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NS; ++q) v[q] = (sh[q][0] + sh[q][1]) + (sh[q][2] + sh[q][3]);
+    int q = NP;
+#pragma unroll
+    for (int a = 0; a < NP; ++a) {
+      h[a] = v[a];
+#pragma unroll
+      for (int b = 0; b < a; ++b) h[a] -= v[q++] * h[b];
+      if (blockIdx.x == 0 && tid == 0) st->H[(k0 + a) * kMaxM + i] = h[a];
+    }
+  } else {
+#pragma unroll
+    for (int a = 0; a < NP; ++a) h[a] = st->H[(k0 + a) * kMaxM + i];
+  }
+  double sp[NP], sn[NN + 1];
+#pragma unroll
+  for (int a = 0; a < NP; ++a) sp[a] = st->vscale[k0 + a];
+#pragma unroll
+  for (int a = 0; a < NN; ++a) sn[a] = st->vscale[k0 + NP + a];
+  double acc[NO];
+#pragma unroll
+  for (int q = 0; q < NO; ++q) acc[q] = 0.0;
+  auto elem = [&](VT we, const VT (&p)[NP], const VT (&x)[NN + 1]) {
+    double wv = (double)we;
+#pragma unroll
+    for (int a = 0; a < NP; ++a) wv = wv + (-h[a]) * ((double)p[a] * sp[a]);
+    const VT r = (VT)wv;
+    wv = (double)r;
+    if constexpr (NN == 0) {
+      acc[0] += wv * wv;
+    } else {
+      double y[NN];
+      int q = NN;
+#pragma unroll
+      for (int a = 0; a < NN; ++a) {
+        y[a] = (double)x[a] * sn[a];
+        acc[a] += y[a] * wv;
+#pragma unroll
+        for (int b = 0; b < a; ++b) acc[q++] += y[a] * y[b];
+      }
+    }
+    return r;
+  };
+  const long stride = (long)gridDim.x * blockDim.x;
+  const long gid = blockIdx.x * (long)blockDim.x + tid;
+  constexpr int W = PK ? Pk<VT>::W : 1;
+  const long nc = n / W;
+  // U turns of the grid-stride loop at a time, all loads first
+  constexpr int U = NP + NN >= 5 ? 1 : NP + NN >= 3 ? 2 : 4;
+  auto turns = [&](long c0, auto chk) {
+    constexpr bool CHK = decltype(chk)::value;
+    Pk<VT> wl[U], pl[U][NP], xl[U][NN + 1];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const long c = c0 + u * stride;
+      if (CHK && c >= nc) break;
+      auto ld = [&](const VT* v) {
+        if constexpr (PK) {
+          return ldpk(v, c);
+        } else {
+          Pk<VT> r;
+          r.v[0] = v[c];
+          return r;
+        }
+      };
+      wl[u] = ld(w);
+#pragma unroll
+      for (int a = 0; a < NP; ++a) pl[u][a] = ld((const VT*)vs.prev[a]);
+#pragma unroll
+      for (int a = 0; a < NN; ++a) xl[u][a] = ld((const VT*)vs.next[a]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const long c = c0 + u * stride;
+      if (CHK && c >= nc) break;
+#pragma unroll
+      for (int j = 0; j < W; ++j) {
+        VT p[NP], x[NN + 1];
+#pragma unroll
+        for (int a = 0; a < NP; ++a) p[a] = pl[u][a].v[j];
+#pragma unroll
+        for (int a = 0; a < NN; ++a) x[a] = xl[u][a].v[j];
+        wl[u].v[j] = elem(wl[u].v[j], p, x);
+      }
+      if constexpr (PK) stpk(w, c, wl[u]);
+      else w[c] = wl[u].v[0];
+    }
+  };
+  long c = gid;
+  for (; c + (U - 1) * stride < nc; c += U * stride) turns(c, std::false_type{});
+  if (c < nc) turns(c, std::true_type{});
+  if constexpr (PK) {  // the n mod W last elements
+    const long e = nc * W + gid;
+    if (e < n) {
+      VT p[NP], x[NN + 1];
+#pragma unroll
+      for (int a = 0; a < NP; ++a) p[a] = ((const VT*)vs.prev[a])[e];
+#pragma unroll
+      for (int a = 0; a < NN; ++a) x[a] = ((const VT*)vs.next[a])[e];
+      w[e] = elem(w[e], p, x);
+    }
+  }
+  block_reduce_store<NO>(acc, partial, blockIdx.x, tid, 256, kMgsStride);
+}
+
+int mgs_blocks(long n) { return std::min(blas_blocks(n), 512); }
+
+template <typename VT, bool PK>
+static void mgs_go(hipStream_t s, long n, VT* w, const MgsVecs& v, int np, int nn, int k0, int i,
+                   KState* st, double* partial, const double* hsrc) {
+  const dim3 grid(mgs_blocks(n)), wg(256);
+#define MGS(P, N)                                                                            \
+  if (np == P && nn == N) {                                                                  \
+    hipLaunchKernelGGL((k_mgs<VT, PK, P, N>), grid, wg, 0, s, n, w, v, k0, i, st, partial,   \
+                       hsrc);                                                                \
+    return;                                                                                  \
+  }
+  // a block that is not full is the last one
+  MGS(1, 0) MGS(1, 1) MGS(1, 2) MGS(1, 3) MGS(2, 0) MGS(3, 0) MGS(3, 1) MGS(3, 2) MGS(3, 3)
+#undef MGS
+}
+
+void launch_mgs(hipStream_t s, long n, int vt, void* const* vs, int k0, int np, int nn, int i,
+                KState* st, double* partial, const double* hsrc) {
+  static_assert(kMgsBlock == 3, "the combinations of mgs_go");
+  void* const w = vs[i + 1];
+  MgsVecs v{};
+  bool pk = al16(w);
+  for (int a = 0; a < np; ++a) pk = al16(v.prev[a] = vs[k0 + a]) && pk;
+  for (int a = 0; a < nn; ++a) pk = al16(v.next[a] = vs[k0 + np + a]) && pk;
+  if (vt == 0) {
+    if (pk) mgs_go<double, true>(s, n, (double*)w, v, np, nn, k0, i, st, partial, hsrc);
+    else mgs_go<double, false>(s, n, (double*)w, v, np, nn, k0, i, st, partial, hsrc);
+  } else {
+    if (pk) mgs_go<float, true>(s, n, (float*)w, v, np, nn, k0, i, st, partial, hsrc);
+    else mgs_go<float, false>(s, n, (float*)w, v, np, nn, k0, i, st, partial, hsrc);
   }
 }
 

@@ -240,13 +240,18 @@ void launch_bicg_update(hipStream_t s, long n, int vt, void* x, const void* ph, 
                         void* r, const void* t, const void* rt, const KState* st,
                         double* partial, const KTail& tail = KTail(),
                         const KTail& fold = KTail());
-// (F)GMRES modified Gram-Schmidt step: w -= H[k-1][i]*vscale[k-1]*v_{k-1} (k>0); then
-// q0 = w.v_k (k<=i) or w.w (k==i+1), into partial slot 0 of `partial`.  hsrc: null (H[k-1][i]
-// is in the state), or the previous step's partial products, whose sum is H[k-1][i]
-// (recorded in the state by workgroup 0).
-void launch_mgs(hipStream_t s, long n, int vt, void* w, const void* vprev, const void* vk,
-                int k, int i, KState* st, double* partial, int chk_done = 0,
-                const double* hsrc = nullptr);
+// One pass of the modified Gram-Schmidt of Arnoldi step i on w = vs[i + 1]: removes the np
+// projections on vs[k0].. (basis vector k is vs[k] * vscale[k]) and forms the sums with the nn
+// vectors after them, or w.w (nn = 0), at `partial`, mgs_blocks partial sums each.  hsrc: null
+// (np = 1, H[k0][i] in the state), or the sums of the pass before, which give the H[k0..][i]
+// (recorded in the state by workgroup 0).  launch_gm_dot: the sum w.w, or w.v_0, into slot 0.
+// Basis vectors a modified Gram-Schmidt pass takes at a time; stride of its partial sums.
+constexpr int kMgsBlock = 3, kMgsStride = 1024;
+int mgs_blocks(long n);
+void launch_gm_dot(hipStream_t s, long n, int vt, const void* w, const void* v0, KState* st,
+                   double* partial, int chk_done);
+void launch_mgs(hipStream_t s, long n, int vt, void* const* vs, int k0, int np, int nn, int i,
+                KState* st, double* partial, const double* hsrc);
 // x += sum_{q<nR} y_q * Z_q  (Z_q = z vectors, FGMRES) with optional scale vscale (GMRES).
 void launch_gmres_update(hipStream_t s, long n, int vt, void* x, void* const* zs, int m,
                          int use_vscale, const KState* st);

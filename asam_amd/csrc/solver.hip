@@ -581,33 +581,33 @@ struct Enq {
     c->counts[2]++;
     fin(FIN_GM_LAST, 1, blas_blocks(c->n), 0, i);
   }
-  void mgs(int vt, void* w, const void* vprev, const void* vk, int k, int i, int chk = 0) {
+  // w.w, or with v0 the product with the first basis vector
+  void gm_dot(int vt, const void* w, const void* v0, int chk = 0) {
     const double ws = vt ? 4 : 8, nv = (double)c->n;
-    double vecs = (k > 0 ? 3 : 1) + (k == i + 1 ? 0 : 1);
-    timed(4 + vt, vecs * nv * ws,
-          [&] { launch_mgs(s, c->n, vt, w, vprev, vk, k, i, c->st, c->partial, chk); });
+    timed(4 + vt, (v0 ? 2 : 1) * nv * ws,
+          [&] { launch_gm_dot(s, c->n, vt, w, v0, c->st, c->partial, chk); });
     c->counts[2]++;
   }
-  // Steps k = 1..i+1 of the modified Gram-Schmidt chain of Arnoldi step i (w = vs[i+1]),
-  // H(0,i) already in the state.  Step k >= 2 sums the previous step's partial products
-  // itself (the same fixed order in every workgroup), so only the last step ends in a
-  // finalize; the steps alternate between partial slots 2 and 3.
+  // The modified Gram-Schmidt of Arnoldi step i (w = vs[i+1]), H(0,i) already in the state:
+  // vector 0, then kMgsBlock vectors a pass.  A pass sums the previous one's partial products
+  // itself (the same fixed order in every workgroup), so only the last ends in a finalize;
+  // the passes alternate between partial slots 2 and 3.
   void mgs_chain(int vt, void* const* vs, int i) {
     const double ws = vt ? 4 : 8, nv = (double)c->n;
     const double* prev = nullptr;
     int slot = 2;
-    for (int k = 1; k <= i + 1; ++k) {
-      const bool self = k == i + 1;
+    for (int k0 = 0, np = 1; k0 <= i;) {
+      const int nn = std::min(kMgsBlock, i + 1 - (k0 + np));
       double* out = c->partial + (long)slot * kRedBlocks;
-      timed(4 + vt, (self ? 3 : 4) * nv * ws, [&] {
-        launch_mgs(s, c->n, vt, vs[i + 1], vs[k - 1], self ? nullptr : vs[k], k, i, c->st, out,
-                   0, prev);
-      });
+      timed(4 + vt, (2 + np + nn) * nv * ws,
+            [&] { launch_mgs(s, c->n, vt, vs, k0, np, nn, i, c->st, out, prev); });
       c->counts[2]++;
       prev = out;
       slot ^= 1;
+      k0 += np;
+      np = nn;
     }
-    fin(FIN_GM_LAST, 1, blas_blocks(c->n), 0, i, 0, 0, prev);
+    fin(FIN_GM_LAST, 1, mgs_blocks(c->n), 0, i, 0, 0, prev);
   }
 };
 
@@ -814,7 +814,7 @@ static int solve_gmres_fp64(asam_sound_ctx* c, int tr, int flexible, int classic
       else
         e.apply(0, 0, 0, 0, x, c->gtmp, b, nullptr, nullptr, 0, &st->done);
       e.line(0, LINE_PLAIN, c->gtmp, nullptr, nullptr, c->gv[0], nullptr, &st->done);
-      e.mgs(0, c->gv[0], nullptr, nullptr, 0, -1, 1);
+      e.gm_dot(0, c->gv[0], nullptr, 1);
       e.fin(FIN_GM_INIT, 1, blas_blocks(n));
     }
     for (int i = 0; i < m; ++i) {
@@ -828,7 +828,7 @@ static int solve_gmres_fp64(asam_sound_ctx* c, int tr, int flexible, int classic
         e.apply(0, 0, 0, 0, c->gv[i], c->gtmp, nullptr, nullptr, nullptr, 0, &st->cycle_done);
         e.line(0, LINE_PLAIN, c->gtmp, nullptr, nullptr, c->gv[i + 1], &st->vscale[i],
                &st->cycle_done);
-        e.mgs(0, c->gv[i + 1], nullptr, c->gv[0], 0, i);
+        e.gm_dot(0, c->gv[i + 1], c->gv[0]);
         e.fin(FIN_GM_H, 1, blas_blocks(n), 0, i);
       }
       if (classical) {
