@@ -140,8 +140,8 @@ struct KEnsLine {
   int kl;  // levels staged in LDS (the rest through the output vector)
 };
 
-template <int NP, int MODE, int LDS, int P, int HV, typename CT, typename VT>
-__global__ __launch_bounds__(64 * HV) void k_ens_line(KEnsLine<CT, VT> e) {
+template <int NP, int MODE, int LDS, int P, typename CT, typename VT>
+__global__ __launch_bounds__(64) void k_ens_line(KEnsLine<CT, VT> e) {
   extern __shared__ unsigned char lds_raw[];
   CT* stage = reinterpret_cast<CT*>(lds_raw);
   const int nb8 = gridDim.x >> 3, per = (e.ntiles + 7) >> 3;
@@ -165,9 +165,9 @@ __global__ __launch_bounds__(64 * HV) void k_ens_line(KEnsLine<CT, VT> e) {
     a.kl = e.kl;
     const int lt = g - M.lt0;
     double acc[1] = {0.0};
-    line_tile<NP, 0, MODE, LDS, P, HV, CT, VT>(a, lt % M.lgx, lt / M.lgx, M.lgx, stage, acc);
+    line_tile<NP, 0, MODE, LDS, P, 1, CT, VT>(a, lt % M.lgx, lt / M.lgx, M.lgx, stage, acc);
     if constexpr (MODE == LINE_BICG_S) {
-      block_reduce_store<1>(acc, e.partial + (long)e.qslot * e.pstride, g, threadIdx.x, 64 * HV,
+      block_reduce_store<1>(acc, e.partial + (long)e.qslot * e.pstride, g, threadIdx.x, 64,
                             e.pstride);
       __syncthreads();
     }
@@ -336,7 +336,6 @@ struct asam_ens_ctx {
   double* partial = nullptr;
   long pstride = 0, pcap = 0;
   int *tA = nullptr, *tL = nullptr, *tB = nullptr;
-  int halves = 1;  // wavefronts per tile of the line solve, by the tiles of all members
   int abx = 256;   // columns per apply tile
   int nA = 0, nL = 0, nB = 0;
   long capA = 0, capL = 0, capB = 0;
@@ -418,7 +417,7 @@ static Geom member_geom(const asam_ens_ctx* c, int m) {
   g.fa = q.fac_anela;
   g.tune = Tuning();
   g.tune.line_tiled = 1;
-  g.halves = c->halves;
+  g.halves = 1;
   return g;
 }
 
@@ -601,13 +600,9 @@ void apply_inner(asam_ens_ctx* c, float* x, float* y, const float* u) {
 
 template <int NP, int MODE, int LDS, int P>
 void line_go(asam_ens_ctx* c, const KEnsLine<float, float>& e, size_t lds) {
-  const dim3 grid(grid_for(c->nL, c->tune.line_pf, c->ncu));
-  if (c->halves == 2)
-    hipLaunchKernelGGL((k_ens_line<NP, MODE, LDS, P, 2, float, float>), grid, dim3(128), lds,
-                       c->stream, e);
-  else
-    hipLaunchKernelGGL((k_ens_line<NP, MODE, LDS, P, 1, float, float>), grid, dim3(64), lds,
-                       c->stream, e);
+  hipLaunchKernelGGL((k_ens_line<NP, MODE, LDS, P, float, float>),
+                     dim3(grid_for(c->nL, c->tune.line_pf, c->ncu)), dim3(64), lds, c->stream,
+                     e);
 }
 
 template <int NP, int MODE>
@@ -617,8 +612,8 @@ void line_inner(asam_ens_ctx* c, const float* src, float* p, const float* v, flo
   e.c = c->c32; e.mem = c->md; e.tmem = c->tL; e.ntiles = c->nL;
   e.src = src; e.p = p; e.v = v; e.out = out; e.st = c->st;
   e.partial = c->partial; e.pstride = c->pstride; e.qslot = qslot;
-  e.kl = lds_levels(c->maxnz, NP, sizeof(float), lds_budget_for(c->tune.line_lds), c->halves);
-  const size_t lds = (size_t)e.kl * c->halves * 64 * NP * sizeof(float);
+  e.kl = lds_levels(c->maxnz, NP, sizeof(float), lds_budget_for(c->tune.line_lds), 1);
+  const size_t lds = (size_t)e.kl * 64 * NP * sizeof(float);
   const bool use = e.kl > 0;
   if (use) {
     if (c->tune.line_window == 8) line_go<NP, MODE, 1, 8>(c, e, lds);
@@ -793,7 +788,6 @@ extern "C" int asam_ens_create(asam_ens_ctx** out, int nmem, const asam_sound_gr
   if (np1 != 1 && np1 != 2) return ASAM_E_INVALID;
   long Ntot = 0, Ftot = 0;
   int maxnz = 0;
-  long tiles = 0;
   for (int m = 0; m < nmem; ++m) {
     const asam_sound_grid& q = grids[m];
     if (q.nx < 1 || q.ny < 1 || q.nz < 1 || q.np1 != np1 || q.grad_full != grids[0].grad_full)
@@ -804,7 +798,6 @@ extern "C" int asam_ens_create(asam_ens_ctx** out, int nmem, const asam_sound_gr
     g.tune.line_tiled = 1;
     Ntot += g.N;
     Ftot += fac_cells(g);
-    tiles += line_blocks(g);
     maxnz = std::max(maxnz, q.nz);
   }
   if (Ntot > (1L << 33)) return ASAM_E_INVALID;
@@ -813,7 +806,6 @@ extern "C" int asam_ens_create(asam_ens_ctx** out, int nmem, const asam_sound_gr
   c->nmem = nmem; c->np1 = np1; c->grad_full = grids[0].grad_full;
   c->grids.assign(grids, grids + nmem);
   c->Ntot = Ntot; c->Ftot = Ftot; c->n = Ntot * np1; c->maxnz = maxnz;
-  c->halves = line_halves(tiles);
   c->ready.assign(nmem, 0);
   c->mh.resize(nmem);
   long off = 0, foff = 0;

@@ -166,8 +166,9 @@ void launch_gm_dot(hipStream_t s, long n, int vt, const void* w, const void* v0,
 // forms the products of the result with the NN vectors after them, or w.w when none is left
 // (NN = 0).  Taking kMgsBlock vectors at a time moves 2 + 2/kMgsBlock vectors per projection
 // instead of 4: FP64 256x256x64 one component, ten steps of a restart cycle, 55 launches of
-// 16.8 us (0.92 ms) before, 28 launches in 0.63 ms together now (7 to 10 TB/s).  The projections stay those of the
-// modified method: with d_a = v_a.w before the block and g_ab = v_a.v_b,
+// 16.8 us (0.92 ms) before, 28 launches in 0.63 ms together now (7 to 10 TB/s).  The
+// projections stay those of the modified method: with d_a = v_a.w before the block and
+// g_ab = v_a.v_b,
 //   h_a = d_a - sum over b < a of g_ab h_b,
 // where the g_ab, of rounding size, come from the same pass as the d_a.
 //

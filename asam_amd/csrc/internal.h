@@ -75,7 +75,7 @@ struct Geom {
   int nx, ny, nz, np1;
   long N;      // cells
   double fa;   // FacAnela
-  int halves;  // wavefronts per tile of the line solve (line_halves)
+  int halves;  // wavefronts per tile of the FP64 line solve (line_halves)
   Tuning tune;
 };
 
@@ -89,15 +89,16 @@ __host__ __device__ inline long fac_index(const Geom& g, int i, int j, int k) {
   }
   return i + (long)g.nx * (j + (long)g.ny * k);
 }
-// Whether the columns of a grid (or of all members of an ensemble) of `tiles` 64-column tiles
-// are eliminated from both ends (Geom::halves = 2), by two wavefronts per tile: up to two
-// tiles per compute unit.  BiCGStab solves, us from the bottom / from both ends (the better
-// window and cache policy of each):
+// Whether the FP64 factors of a grid of `tiles` 64-column tiles eliminate the columns from both
+// ends (Geom::halves = 2), by two wavefronts per tile: up to two tiles per compute unit.
+// BiCGStab solves, us from the bottom / from both ends (the better window and cache policy of
+// each):
 //   tiles            64        192       291       480         600         1024
 //   2x2 FP64      466/427   600/565   711/690   2112/2124   2696/2790   5222/5231
-//   2x2 mixed     436/389   505/473   578/555   1287/1276   1619/1602   2750/2784
 //   1-comp. FP64  318/293   434/405   491/471   1114/1119   1350/1337   2603/2657
-//   1-comp. mixed 325/295   354/325   394/373    866/846     962/944    1534/1549
+// The FP32 factors of a mixed solve always go from the bottom up (there 64 tiles of 2x2 blocks
+// would take 389 us for 436): the other order rounds every entry differently, and that moves a
+// solution refined to 1e-8 by up to 2.4e-9 of its norm (128x128x64).
 constexpr int line_halves(long tiles) { return tiles <= 512 ? 2 : 1; }
 // Words per cell of the line solve's blocks towards the previous level of the elimination:
 // L_k, and with elimination from both ends U_k from the middle nz/2 up.  A 2x2 block couples two levels through one
@@ -170,6 +171,7 @@ void launch_coef(hipStream_t s, const Geom& g, int grad_full, double beta0_dt, d
                  const double* dx, const double* dy, const double* dz, const double* thu,
                  const double* thv, const double* thw, Coef<double>& c);
 void launch_factor(hipStream_t s, const Geom& g, Coef<double>& c);
+void launch_factors(hipStream_t s, const Geom& g, Coef<double>& c64, Coef<float>& c32);
 void launch_convert(hipStream_t s, const Geom& g, const Coef<double>& c64, Coef<float>& c32);
 
 // ------------------------------------------------------------------ apply

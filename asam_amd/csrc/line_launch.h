@@ -80,17 +80,21 @@ static bool line_nontemporal(const Geom& g) {
 template <int NP, int TR, int LDS, int P, typename CT, typename VT>
 static void line_launch(hipStream_t s, const Geom& g, const KLine<CT, VT>& a, int mode,
                         size_t lds) {
-  if (line_nontemporal<NP, CT>(g)) {
-    if (g.halves == 2) line_mode<NP, TR, LDS, P, 2, 1, CT, VT>(s, g, a, mode, lds);
-    else line_mode<NP, TR, LDS, P, 1, 1, CT, VT>(s, g, a, mode, lds);
-  } else {
-    if (g.halves == 2) line_mode<NP, TR, LDS, P, 2, 0, CT, VT>(s, g, a, mode, lds);
-    else line_mode<NP, TR, LDS, P, 1, 0, CT, VT>(s, g, a, mode, lds);
+  const bool nt = line_nontemporal<NP, CT>(g);
+  if constexpr (sizeof(CT) == 8) {
+    if (g.halves == 2) {
+      if (nt) line_mode<NP, TR, LDS, P, 2, 1, CT, VT>(s, g, a, mode, lds);
+      else line_mode<NP, TR, LDS, P, 2, 0, CT, VT>(s, g, a, mode, lds);
+      return;
+    }
   }
+  if (nt) line_mode<NP, TR, LDS, P, 1, 1, CT, VT>(s, g, a, mode, lds);
+  else line_mode<NP, TR, LDS, P, 1, 0, CT, VT>(s, g, a, mode, lds);
 }
 
 template <int NP, int TR, typename CT, typename VT>
 static void line_t(hipStream_t s, const Geom& g, const Coef<CT>& c, const LineReq& r) {
+  const int halves = sizeof(CT) == 8 ? g.halves : 1;
   KLine<CT, VT> a;
   a.c = c; a.nx = g.nx; a.ny = g.ny; a.nz = g.nz; a.tiled = g.tune.line_tiled;
   a.src = (const VT*)r.src; a.p = (VT*)r.p; a.v = (const VT*)r.v; a.out = (VT*)r.out;
@@ -98,19 +102,19 @@ static void line_t(hipStream_t s, const Geom& g, const Coef<CT>& c, const LineRe
   a.qslot = r.qslot;
   a.fold = r.fold;
   a.kl = r.use_lds ? lds_levels(g.nz, NP, sizeof(CT), lds_budget_for(g.tune.line_lds),
-                                g.halves)
+                                halves)
                    : 0;
-  const size_t lds = (size_t)a.kl * g.halves * 64 * NP * sizeof(CT);
+  const size_t lds = (size_t)a.kl * halves * 64 * NP * sizeof(CT);
   const bool use_lds = a.kl > 0;
   // Default window: 8 levels, but 4 for 2x2 blocks with two wavefronts per tile once a
-  // compute unit has two tiles: another tile's loads then hide a window's latency.  BiCGStab
-  // solves, us with 4 / 8 levels: two wavefronts, 2x2 mixed 64x64x40 394/389, 128x128x64
-  // 1017/1036, 2x2 FP64 128x128x32 585/613, 130x97x40 690/701, one component FP64 64x64x40
-  // 299/293, 192x128x50 1041/1044; one wavefront, 2x2 FP64 201x150x50 2702/2696, 256x192x56
-  // 4144/4114, mixed 256x256x64 2802/2750, one component FP64 256x256x64 2724/2603.
+  // compute unit has a tile: another tile's loads then hide a window's latency.  BiCGStab
+  // solves, us with 4 / 8 levels: two wavefronts, 2x2 FP64 128x128x32 585/613, 130x97x40
+  // 690/701, 64x64x40 427/428, one component FP64 64x64x40 299/293, 192x128x50 1041/1044; one
+  // wavefront, 2x2 FP64 201x150x50 2702/2696, 256x192x56 4144/4114, mixed 256x256x64
+  // 2802/2750, one component FP64 256x256x64 2724/2603.
   const int P = g.tune.line_window > 0
                     ? g.tune.line_window
-                    : (NP == 2 && g.halves == 2 && line_blocks(g) >= 256 ? 4 : 8);
+                    : (NP == 2 && halves == 2 && line_blocks(g) >= 256 ? 4 : 8);
   if (use_lds) {
     if (P >= 8) line_launch<NP, TR, 1, 8, CT, VT>(s, g, a, r.mode, lds);
     else if (P >= 4) line_launch<NP, TR, 1, 4, CT, VT>(s, g, a, r.mode, lds);

@@ -254,7 +254,7 @@ __global__ __launch_bounds__(128) void k_factor(Geom g, Coef<double> c) {
       W[0] = meets || t == 0.0 ? 0.0 : N[0] / t;
       c.pt[fi] = ti;
       c.pw[fi] = W[0];
-      if (half || k > 0) c.pl[fi] = half ? b.u3[0] : b.l3[0];
+      if (mid == nz || half || k > 0) c.pl[fi] = half ? b.u3[0] : b.l3[0];
       if (meets && mid > 0) c.pl[fac_index(g, i, j, 0)] = b.l3[0];
       return;
     }
@@ -273,7 +273,7 @@ __global__ __launch_bounds__(128) void k_factor(Geom g, Coef<double> c) {
       *reinterpret_cast<double2*>(c.pt + 4 * fi + q) = make_double2(T[q], T[q + 1]);
       *reinterpret_cast<double2*>(c.pw + 4 * fi + q) = make_double2(W[q], W[q + 1]);
     }
-    if (half || k > 0)
+    if (mid == nz || half || k > 0)
       for (int q = 0; q < 3; ++q) c.pl[3 * fi + q] = half ? b.u3[q] : b.l3[q];
     if (meets && mid > 0) {
       const long f0 = fac_index(g, i, j, 0);
@@ -320,6 +320,16 @@ void launch_convert(hipStream_t s, const Geom& g, const Coef<double>& c64, Coef<
   cv(c64.gz, c32.gz, N); cv(c64.vol, c32.vol, N); cv(c64.dut, c32.dut, N);
   cv(c64.pl, c32.pl, PL); cv(c64.pt, c32.pt, P); cv(c64.pw, c32.pw, P);
   if (c32.pkz) hipLaunchKernelGGL(k_pack_z, dim3((N + 255) / 256), dim3(256), 0, s, N, c32);
+}
+
+// Line factors of both precisions, and the FP32 copies of the operator.  The FP32 factors are
+// those of the elimination from the bottom up (see line_halves).
+void launch_factors(hipStream_t s, const Geom& g, Coef<double>& c64, Coef<float>& c32) {
+  Geom up = g;
+  up.halves = 1;
+  launch_factor(s, up, c64);
+  launch_convert(s, g, c64, c32);
+  if (g.halves == 2) launch_factor(s, g, c64);
 }
 
 // Dead cells of the residual form: the apply's own test (march_tile), same operand order.

@@ -173,8 +173,7 @@ extern "C" int asam_sound_set_tuning(asam_sound_ctx* c, const asam_sound_tuning*
   c->g.tune = nt;
   if (relayout && c->ready) {  // the line factors live in the layout the tuning names
     HIPCHK(c, hipSetDevice(c->device));
-    launch_factor(c->stream, c->g, c->c64);
-    launch_convert(c->stream, c->g, c->c64, c->c32);
+    launch_factors(c->stream, c->g, c->c64, c->c32);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
   }
@@ -347,8 +346,7 @@ static int setup_common(asam_sound_ctx* c, const double* FU, const double* FV, c
   }
   launch_coef(s, g, c->grid.grad_full, c->grid.beta0_dt, c->grid.grav, dFU, dFV, dFW, dV, ddx,
               ddy, ddz, thu, thv, thw, c->c64);
-  launch_factor(s, g, c->c64);
-  launch_convert(s, g, c->c64, c->c32);
+  launch_factors(s, g, c->c64, c->c32);
   launch_dead_mask(s, g, c->c64, c->dead);
   HIPCHK(c, hipGetLastError());
   HIPCHK(c, hipStreamSynchronize(s));
