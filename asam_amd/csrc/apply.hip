@@ -43,10 +43,12 @@ static ApplyShape tile_shape(const Geom& g, int bx, int rows, int kp) {
 
 // The default shape (variant 3, two rows per thread): the launch ends with the compute unit
 // that has most to do, so take the tile for which that is least.  A unit with n tiles of kp
-// planes takes n (kp + 1) plane times: kp + 1 because a tile starts by loading the planes
-// around its first one; n no less than the tiles a unit needs at once to be busy, two, and
-// three for one component in FP32, which moves the fewest bytes.  A plane time is the
-// wavefronts of the tile that have columns at all; 32 columns (two stacked row blocks per
+// planes and w wavefronts that have columns at all takes n w (kp + 2): a tile
+// starts by loading the planes around its first one (with kp + 1 64x64x64 took tiles of one
+// plane, 2x2 mixed 851 us for 801); n w no less than the wavefronts a unit
+// needs at once to be busy, six, and nine for one component in FP32, which moves the fewest
+// bytes (with a floor on n alone 128x128x64 took tiles of 256 columns, half of them empty, 2x2
+// mixed 1085 us for 1048).  32 columns (two stacked row blocks per
 // wavefront) cost a tenth more.  Against 128 columns and about 512 workgroups for every grid,
 // BiCGStab solves, us before / after: 201x150x50 one component FP64 1360/1201, 2x2 FP64
 // 2790/2480, 2x2 mixed 1638/1454; 256x192x56 2x2 FP64 4132/3714, one component mixed
@@ -54,7 +56,7 @@ static ApplyShape tile_shape(const Geom& g, int bx, int rows, int kp) {
 // mixed 579/510; 512x512x96 one component mixed 9118/8518; 256x256x64 2x2: the same shape.
 static ApplyShape balanced_shape(const Geom& g, int fp32) {
   constexpr int kCUs = 256;
-  const int busy = g.np1 == 1 && fp32 ? 3 : 2;
+  const long busy = g.np1 == 1 && fp32 ? 9 : 6;
   ApplyShape best{};
   long least = 0;
   for (int bx : {128, 256, 64, 32}) {
@@ -68,8 +70,8 @@ static ApplyShape balanced_shape(const Geom& g, int fp32) {
       if (kp == last) continue;
       last = kp;
       const ApplyShape a = tile_shape(g, bx, rows, kp);
-      const long per = std::max((a.nblocks + kCUs - 1) / kCUs, busy);
-      const long cost = per * waves * (kp + 1) * (bx == 32 ? 11 : 10);
+      const long per = std::max((long)((a.nblocks + kCUs - 1) / kCUs) * waves, busy);
+      const long cost = per * (kp + 2) * (bx == 32 ? 11 : 10);
       if (a.nblocks <= kRedBlocks && (least == 0 || cost < least)) {
         least = cost;
         best = a;

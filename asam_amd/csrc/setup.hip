@@ -231,30 +231,41 @@ __device__ __forceinline__ LineBlocks line_blocks_at(const Geom& g, const Coef<d
   return b;
 }
 
-// 64 columns per workgroup, one wavefront for each half; the upper one does the middle level
-// when the lower one has left its last w in LDS.
-__global__ __launch_bounds__(128) void k_factor(Geom g, Coef<double> c) {
+// 64 columns per workgroup; with elimination from both ends one wavefront for each half, the
+// upper one doing the middle level when the lower one has left its last w in LDS.  The FP32
+// factors (f, if any) are those of the elimination from the bottom up (see line_halves),
+// written with the FP64 ones where these are the same, else by the second row of the grid.
+// Bound by the chain of a column: the blocks of the next level are formed while this one is
+// eliminated.
+__global__ __launch_bounds__(128) void k_factor(Geom g, Coef<double> c, Coef<float> f) {
   __shared__ double wl[4][64];
   const int lane = threadIdx.x & 63, half = threadIdx.x >> 6;
   const long col = blockIdx.x * 64L + lane;
   const bool on = col < (long)g.nx * g.ny;
   const int i = on ? (int)(col % g.nx) : 0, j = on ? (int)(col / g.nx) : 0;
-  const int nz = g.nz, mid = g.halves == 2 ? nz / 2 : nz;
+  const bool two = g.halves == 2 && blockIdx.y == 0;
+  const bool w64 = blockIdx.y == 0, w32 = f.pl && (g.halves == 1 || blockIdx.y == 1);
+  const int nz = g.nz, mid = two ? nz / 2 : nz;
+  if (!two && half) return;
+  auto put = [&](double* p, float* q, long e, double v) {
+    if (w64) p[e] = v;
+    if (w32) q[e] = (float)v;
+  };
   double W[4] = {0, 0, 0, 0};
   // level k: t = D - (block towards the previous level) W [- L_m (lower half's W)]
-  auto level = [&](int k, bool meets) {
-    const LineBlocks b = line_blocks_at(g, c, i, j, k);
+  auto level = [&](const LineBlocks& b, int k, bool meets) {
     const double* const A = half ? b.U : b.L;   // towards the previous level
     const double* const N = half ? b.L : b.U;   // towards the next one
     const long fi = fac_index(g, i, j, k);
+    const bool lower = !two || half || k > 0;   // else the place is L_m's
     if (g.np1 == 1) {
       double t = b.D[0] - A[0] * W[0];
       if (meets) t -= b.L[0] * wl[0][lane];
       const double ti = t == 0.0 ? 0.0 : 1.0 / t;
       W[0] = meets || t == 0.0 ? 0.0 : N[0] / t;
-      c.pt[fi] = ti;
-      c.pw[fi] = W[0];
-      if (mid == nz || half || k > 0) c.pl[fi] = half ? b.u3[0] : b.l3[0];
+      put(c.pt, f.pt, fi, ti);
+      put(c.pw, f.pw, fi, W[0]);
+      if (lower) put(c.pl, f.pl, fi, half ? b.u3[0] : b.l3[0]);
       if (meets && mid > 0) c.pl[fac_index(g, i, j, 0)] = b.l3[0];
       return;
     }
@@ -269,33 +280,45 @@ __global__ __launch_bounds__(128) void k_factor(Geom g, Coef<double> c) {
     inv22(t, T);
     if (meets) W[0] = W[1] = W[2] = W[3] = 0.0;
     else mul22(T, N, W);
-    for (int q = 0; q < 4; q += 2) {
-      *reinterpret_cast<double2*>(c.pt + 4 * fi + q) = make_double2(T[q], T[q + 1]);
-      *reinterpret_cast<double2*>(c.pw + 4 * fi + q) = make_double2(W[q], W[q + 1]);
+    for (int q = 0; q < 4; ++q) {
+      put(c.pt, f.pt, 4 * fi + q, T[q]);
+      put(c.pw, f.pw, 4 * fi + q, W[q]);
     }
-    if (mid == nz || half || k > 0)
-      for (int q = 0; q < 3; ++q) c.pl[3 * fi + q] = half ? b.u3[q] : b.l3[q];
+    if (lower)
+      for (int q = 0; q < 3; ++q) put(c.pl, f.pl, 3 * fi + q, half ? b.u3[q] : b.l3[q]);
     if (meets && mid > 0) {
       const long f0 = fac_index(g, i, j, 0);
       for (int q = 0; q < 3; ++q) c.pl[3 * f0 + q] = b.l3[q];
     }
   };
+  const int k0 = half ? nz - 1 : 0, dk = half ? -1 : 1, nk = half ? nz - 1 - mid : mid;
+  LineBlocks b{};
   if (on) {
-    if (half == 0)
-      for (int k = 0; k < mid; ++k) level(k, false);
-    else
-      for (int k = nz - 1; k > mid; --k) level(k, false);
+    b = line_blocks_at(g, c, i, j, k0);
+    for (int q = 0; q < nk; ++q) {
+      const int k = k0 + dk * q, kn = k + dk;
+      const LineBlocks next = line_blocks_at(g, c, i, j, kn < nz ? kn : k);
+      level(b, k, false);
+      b = next;
+    }
   }
-  if (g.halves == 1) return;
+  if (!two) return;
   if (half == 0)
     for (int q = 0; q < 4; ++q) wl[q][lane] = W[q];
   __syncthreads();
-  if (on && half) level(mid, true);
+  if (on && half) level(b, mid, true);
 }
 
+static void factor(hipStream_t s, const Geom& g, Coef<double>& c64, const Coef<float>& c32) {
+  const long ncol = (long)g.nx * g.ny;
+  const int rows = g.halves == 2 && c32.pl ? 2 : 1;
+  hipLaunchKernelGGL(k_factor, dim3((ncol + 63) / 64, rows), dim3(64 * g.halves), 0, s, g, c64,
+                     c32);
+}
+
+// The FP64 line factors alone.
 void launch_factor(hipStream_t s, const Geom& g, Coef<double>& c) {
-  long ncol = (long)g.nx * g.ny;
-  hipLaunchKernelGGL(k_factor, dim3((ncol + 63) / 64), dim3(64 * g.halves), 0, s, g, c);
+  factor(s, g, c, Coef<float>());
 }
 
 __global__ void k_cvt(long n, const double* a, float* b) {
@@ -309,7 +332,8 @@ __global__ void k_pack_z(long n, Coef<float> c) {
   reinterpret_cast<float4*>(c.pkz)[i] = make_float4(c.kz[i], c.tz[i], c.gz[i], c.vol[i]);
 }
 
-void launch_convert(hipStream_t s, const Geom& g, const Coef<double>& c64, Coef<float>& c32) {
+static void convert(hipStream_t s, const Geom& g, const Coef<double>& c64, Coef<float>& c32,
+                    bool factors) {
   const long N = g.N, P = (long)g.np1 * g.np1 * fac_cells(g);
   const long PL = (long)lower_words(g.np1) * fac_cells(g);
   auto cv = [&](const double* a, float* b, long n) {
@@ -318,18 +342,20 @@ void launch_convert(hipStream_t s, const Geom& g, const Coef<double>& c64, Coef<
   cv(c64.kx, c32.kx, N); cv(c64.ky, c32.ky, N); cv(c64.kz, c32.kz, N);
   cv(c64.tx, c32.tx, N); cv(c64.ty, c32.ty, N); cv(c64.tz, c32.tz, N);
   cv(c64.gz, c32.gz, N); cv(c64.vol, c32.vol, N); cv(c64.dut, c32.dut, N);
-  cv(c64.pl, c32.pl, PL); cv(c64.pt, c32.pt, P); cv(c64.pw, c32.pw, P);
+  if (factors) {
+    cv(c64.pl, c32.pl, PL); cv(c64.pt, c32.pt, P); cv(c64.pw, c32.pw, P);
+  }
   if (c32.pkz) hipLaunchKernelGGL(k_pack_z, dim3((N + 255) / 256), dim3(256), 0, s, N, c32);
 }
 
-// Line factors of both precisions, and the FP32 copies of the operator.  The FP32 factors are
-// those of the elimination from the bottom up (see line_halves).
+void launch_convert(hipStream_t s, const Geom& g, const Coef<double>& c64, Coef<float>& c32) {
+  convert(s, g, c64, c32, true);
+}
+
+// Line factors of both precisions, and the FP32 copies of the operator.
 void launch_factors(hipStream_t s, const Geom& g, Coef<double>& c64, Coef<float>& c32) {
-  Geom up = g;
-  up.halves = 1;
-  launch_factor(s, up, c64);
-  launch_convert(s, g, c64, c32);
-  if (g.halves == 2) launch_factor(s, g, c64);
+  factor(s, g, c64, c32);
+  convert(s, g, c64, c32, false);
 }
 
 // Dead cells of the residual form: the apply's own test (march_tile), same operand order.
