@@ -7,10 +7,10 @@
 //   natural: the reference's arrays, x fastest: Val(m, 7) column-major for JacTMom and
 //     JacTPot, Val(m, 2) for JacFall; vectors ncomp x m; LU factors ncomp*ncomp x ncell.
 //   skewed (Gauss-Seidel only): level k, y-tile jt of TW columns j, row h = i + jj of
-//     the tile (jj the column within it), 64 entries per row: the cells of one step of a
-//     wavefront whose lanes are the columns (lane l at cell i = step - l) are one contiguous
-//     run.  A matrix holds kCoefWords such runs per row, one after the other.  The skew costs
-//     1 + (TW-1)/X of padding; a step reads whole 128-byte lines.
+//     the tile (jj the column within it), RW entries per row, one per column: the cells of one
+//     step of a wavefront whose lanes are the columns (lane l at cell i = step - l) are one
+//     contiguous run.  A matrix holds kCoefWords such runs per row, one after the other.  The
+//     skew costs 1 + (TW-1)/X of padding, the rows RW/TW (see Dims).
 //
 // The Gauss-Seidel sweep is the reference's lexicographic forward sweep.  Cell (i, j, k)
 // needs the new values of (i-1), (j-1), (k-1) and the old ones of (i+1), (j+1), (k+1), so
@@ -45,7 +45,9 @@ struct Ops {
 struct Dims {
   int nx, ny, nz, X, Y, Z;
   int TW, NJ, HL;         // skewed layout: columns per y-tile, y-tiles, rows per tile and level
-  long m, ncell, slots;   // slots = Z*NJ*HL*64
+  int RW;                 // entries per row: kRow, or for few columns as many, see create
+  int ZW;                 // columns of a boundary record's top level
+  long m, ncell, slots;   // slots = Z*NJ*HL*RW
 };
 
 // Components that go through the sweeps together, one or two per group: two share a matrix
@@ -175,13 +177,18 @@ __device__ __forceinline__ bool gs_plain_diag(double dg) {
 // ------------------------------------------------------------------ skewed layout
 // Slot of cell (i, j, k) within an array of one word per cell: y-tile jt = j / TW, column
 // jj = j - jt*TW, row h = i + jj of the tile's HL = X + TW - 1 rows.
-constexpr int kRow = 64;       // entries of a row of the skewed layout
 constexpr int kCoefWords = 8;  // words per cell of a skewed matrix: see k_skew_coef
+constexpr int kMaxCols = 53;   // columns of a y-tile at most, see kMaxSweeps below
+// Entries of a row of the skewed layout for tiles of 27 columns and more.  Rows of 56 (the most
+// that a tile needs, in whole 128-byte lines) would take less memory and more time: an
+// application at 256x256x64, four components, 1346 us against 1330, a sweep of 101x77x50 with
+// JacFall 42.4 against 41.3.
+constexpr int kRow = 64;
 
 // Place of word q of a cell within a matrix row: the words lie in pairs, so that a lane takes
 // two with one 16-byte load (a wavefront's load costs the address unit the same 16 cycles
 // whatever its width).
-__device__ __forceinline__ constexpr int coef_word(int q) { return (q >> 1) * (2 * kRow) + (q & 1); }
+__device__ __forceinline__ int coef_word(int RW, int q) { return (q >> 1) * (2 * RW) + (q & 1); }
 
 __device__ __forceinline__ long slot_row(const Dims& d, int jt, int h, int k) {
   return ((long)k * d.NJ + jt) * d.HL + h;
@@ -231,10 +238,10 @@ __global__ __launch_bounds__(256) void k_skew_coef(Dims d, const double* __restr
           return in ? val[(long)dq[q] * d.m + i2 + (long)d.X * (j2 + (long)d.Y * k2)] : 0.0;
         },
         [&](int h, int jj, double v) {
-          double* row = w + slot_row(d, jt, h, k) * (kCoefWords * kRow) + 2 * jj;
-          row[coef_word(q)] = v;
+          double* row = w + slot_row(d, jt, h, k) * (kCoefWords * d.RW) + 2 * jj;
+          row[coef_word(d.RW, q)] = v;
           if (q == 6) {
-            row[coef_word(7)] = 1.0 / v;
+            row[coef_word(d.RW, 7)] = 1.0 / v;
             if (!gs_plain_diag(v)) *odd = 1;
           }
         });
@@ -255,7 +262,7 @@ __global__ __launch_bounds__(256) void k_skew_fall(Dims d, const double* __restr
           return k2 < d.Z ? fall[q * d.m + i + (long)d.X * (jt * d.TW + jj + (long)d.Y * k2)] : 0.0;
         },
         [&](int h, int jj, double v) {
-          wf[slot_row(d, jt, h, k) * (2 * kRow) + 2 * jj + q] = v;
+          wf[slot_row(d, jt, h, k) * (2 * d.RW) + 2 * jj + q] = v;
         });
 }
 // A vector to the skewed layout, the NC components of a group together (they lie side by side
@@ -266,7 +273,6 @@ __global__ __launch_bounds__(256) void k_skew_fall(Dims d, const double* __restr
 // now 54 us and 56 us (4.9 TB/s).
 // Grid (y-tiles x runs of kVecH rows, 1, levels x groups).
 constexpr int kVecH = 32;
-constexpr int kMaxCols = 53;  // columns of a y-tile at most, see kMaxSweeps below
 template <int NC>
 __global__ __launch_bounds__(256) void k_skew_vec(Dims d, Groups gr, const double* __restrict__ v,
                                                   double* __restrict__ vs) {
@@ -301,7 +307,7 @@ __global__ __launch_bounds__(256) void k_skew_vec(Dims d, Groups gr, const doubl
   for (int hh = wv; hh < kVecH; hh += 4) {
     const int h = h0 + hh, i = h - lane;
     if (lane < rows && h < d.HL && i >= 0 && i < d.X) {
-      double* const p = dst + (slot_row(d, jt, h, k) * kRow + lane) * NC;
+      double* const p = dst + (slot_row(d, jt, h, k) * d.RW + lane) * NC;
       if constexpr (NC == 2)
         *reinterpret_cast<double2*>(p) = make_double2(t[0][lane][hh], t[1][lane][hh]);
       else
@@ -331,7 +337,7 @@ __global__ __launch_bounds__(256) void k_unskew(Dims d, Groups gr, const double*
     for (int q = 0; q < NH; ++q) {
       const int l = wv + 4 * q - lane, h = i0 + wv + 4 * q;
       const bool in = lane < rows && l >= 0 && l < kVecH && i0 + l < d.X;
-      const double* const p = src + (slot_row(d, jt, h, k) * kRow + lane) * NC;
+      const double* const p = src + (slot_row(d, jt, h, k) * d.RW + lane) * NC;
 #pragma unroll
       for (int n = 0; n < NC; ++n) x[q][n] = 0.0;
       if (in) {
@@ -411,21 +417,21 @@ __global__ __launch_bounds__(256) void k_gs_upart(GsArgs a, Ops ops, double* __r
   if (h >= d.HL || lane >= d.TW || j >= d.Y || i < 0 || i >= d.X) return;
   const long base = g * d.slots * NC + n;
   const double* const x = a.xs + base;
-  const long row = slot_row(d, jt, h, k), e = row * kRow + lane;
+  const long row = slot_row(d, jt, h, k), e = row * d.RW + lane;
   const double* const w =
-      (ops.op[c] == ASAM_TR_MOM ? a.wmom : a.wpot) + row * (kCoefWords * kRow) + 2 * lane;
+      (ops.op[c] == ASAM_TR_MOM ? a.wmom : a.wpot) + row * (kCoefWords * d.RW) + 2 * lane;
   double t = a.bs[base + e * NC];
-  if (i + 1 < d.X) t = t - w[coef_word(0)] * x[(e + kRow) * NC];
+  if (i + 1 < d.X) t = t - w[coef_word(d.RW, 0)] * x[(e + d.RW) * NC];
   if (j + 1 < d.Y) {
     // the next column: in this tile one row on, or the first of the next tile, row i
-    const long e2 = lane + 1 < d.TW ? e + kRow + 1 : slot_row(d, jt + 1, i, k) * kRow;
-    t = t - w[coef_word(1)] * x[e2 * NC];
+    const long e2 = lane + 1 < d.TW ? e + d.RW + 1 : slot_row(d, jt + 1, i, k) * d.RW;
+    t = t - w[coef_word(d.RW, 1)] * x[e2 * NC];
   }
   if (k + 1 < d.Z) {
-    const double xz = x[(e + (long)d.NJ * d.HL * kRow) * NC];
-    t = t - w[coef_word(2)] * xz;
+    const double xz = x[(e + (long)d.NJ * d.HL * d.RW) * NC];
+    t = t - w[coef_word(d.RW, 2)] * xz;
     if (ops.op[c] == ASAM_TR_FALL)
-      t = t - (a.wf[row * (2 * kRow) + 2 * lane + 1] * ops.alpha[c]) * xz;
+      t = t - (a.wf[row * (2 * d.RW) + 2 * lane + 1] * ops.alpha[c]) * xz;
   }
   tw[base + e * NC] = t;
 }
@@ -516,8 +522,10 @@ __device__ __forceinline__ bool any_sentinel(const Val<NC>& v) {
 }
 
 // DIV: divide by the diagonal (a matrix with an unusual one, or JacFall in it) instead of
-// multiplying by its reciprocal.
-template <int NC, int KR, int D, bool FALL, bool DIV, typename OFF>
+// multiplying by its reciprocal.  ROW: entries of a row, 0: as in Dims (the places of a row's
+// pairs then take scalar registers and instructions that constants do not: 1.7% of the launch
+// at 256x256x64, 4.5% at 101x77x50 with JacFall).
+template <int NC, int KR, int D, bool FALL, bool DIV, int ROW, typename OFF>
 __global__ __launch_bounds__(512, 2) void k_gs_tiles(GsArgs a, Ops ops) {
 #pragma clang fp contract(off)
   using V = Val<NC>;
@@ -525,6 +533,7 @@ __global__ __launch_bounds__(512, 2) void k_gs_tiles(GsArgs a, Ops ops) {
   V* const lds = reinterpret_cast<V*>(lds_raw);  // [2][M][KR + 1][kLdsRow], level -1, column -1 first
   __shared__ int s_ticket;
   const Dims& d = a.d;
+  const int RW = ROW ? ROW : d.RW;
   const int lane = threadIdx.x & 63, M = a.M, TW = d.TW, X = d.X;
   const int s = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   constexpr int kWave = (KR + 1) * kLdsRow;
@@ -536,9 +545,11 @@ __global__ __launch_bounds__(512, 2) void k_gs_tiles(GsArgs a, Ops ops) {
   const int g = ticket % a.groups.n, blk = a.order[ticket / a.groups.n];
   const int jt = blk % d.NJ, kb = blk / d.NJ;
   const int nsteps = a.nsteps, steps = (nsteps + PF - 1) / PF * PF;
-  // a record: top level [sweep][lane], last column [sweep][level], NC values each
-  const int zrec = M * TW * NC, yrec = M * KR * NC;
-  const long rec = zrec + yrec, brec = nsteps * rec;
+  // a record: top level [sweep][column], last column [sweep][level], NC values each; a single
+  // tile has no successor in y, and sweep s has its Y columns at lanes s and up
+  const int ZW = d.ZW, zshift = d.NJ == 1 ? 1 : 0;
+  const int zrec = M * ZW * NC, yrec = M * KR * NC;
+  const long rec = zrec + (d.NJ == 1 ? 0 : yrec), brec = nsteps * rec;
   const long nblk = (long)d.NJ * a.NK;
   double* const bnd = a.bnd + g * nblk * brec;
 
@@ -548,8 +559,9 @@ __global__ __launch_bounds__(512, 2) void k_gs_tiles(GsArgs a, Ops ops) {
     int zdst[kZWords];
 #pragma unroll
     for (int q = 0; q < kZWords; ++q) {
-      const int e = lane + 64 * q, w = e / TW;
-      zdst[q] = e < M * TW ? w * kWave + e - w * TW + 1 : kLdsRow - 1;  // or a pad entry
+      const int e = lane + 64 * q, w = e / ZW;
+      // or a pad entry
+      zdst[q] = e < M * ZW ? w * kWave + e - w * (ZW - zshift) + 1 : kLdsRow - 1;
     }
     // the column values, and those of level -1 beside them
     int f = lane, ylast = -2, ydst = (kLdsRow - 1) * NC;
@@ -640,14 +652,14 @@ __global__ __launch_bounds__(512, 2) void k_gs_tiles(GsArgs a, Ops ops) {
     int zsrc[kZWords];
 #pragma unroll
     for (int q = 0; q < kZWords; ++q) {
-      const int e = lane + 64 * q, w = e / TW;
-      zsrc[q] = e < M * TW ? w * kWave + KR * kLdsRow + e - w * TW + 1 : 0;
+      const int e = lane + 64 * q, w = e / ZW;
+      zsrc[q] = e < M * ZW ? w * kWave + KR * kLdsRow + e - w * (ZW - zshift) + 1 : 0;
     }
     const int ye = lane / NC, yw = ye / KR, yr = ye - yw * KR;
     const int ysrc = pub_y ? (yw * kWave + (yr + 1) * kLdsRow + TW) * NC + lane % NC : 0;
     double* out = bnd + blk * brec;
     const int z = M - 1, j = jt * TW - z + lane;
-    const OFF off = ((lane < z ? (OFF)TW : (OFF)d.HL) * kRow + (lane < z ? lane - z + TW : lane - z)) *
+    const OFF off = ((lane < z ? (OFF)TW : (OFF)d.HL) * RW + (lane < z ? lane - z + TW : lane - z)) *
                     (8 * NC);
     double* const xs = a.xs + g * d.slots * NC;
     bool cell[KR];
@@ -677,7 +689,7 @@ __global__ __launch_bounds__(512, 2) void k_gs_tiles(GsArgs a, Ops ops) {
       for (int r = 0; r < KR; ++r) {
         const int k = min(max(kb * KR - z + r, 0), d.Z - 1);
         char* const row =
-            reinterpret_cast<char*>(xs + slot_row(d, jt - 1, T - r - z, k) * (kRow * NC));
+            reinterpret_cast<char*>(xs + slot_row(d, jt - 1, T - r - z, k) * (RW * NC));
         if (cell[r] & ((unsigned)(T - lane - r) < (unsigned)X))
           *reinterpret_cast<V*>(row + off) = L[z * kWave + (r + 1) * kLdsRow + lane + 1];
       }
@@ -702,12 +714,12 @@ __global__ __launch_bounds__(512, 2) void k_gs_tiles(GsArgs a, Ops ops) {
   // tile's first lie in tile jt - 1, TW rows on.
   const OFF rowl = lane < s ? TW : d.HL;
   const int col = lane < s ? lane - s + TW : lane - s;
-  const OFF offw = (rowl * (kCoefWords * kRow) + 2 * col) * 8, offb = (rowl * kRow + col) * (8 * NC);
-  const OFF offf = (rowl * (2 * kRow) + 2 * col) * 8;
+  const OFF offw = (rowl * (kCoefWords * RW) + 2 * col) * 8, offb = (rowl * RW + col) * (8 * NC);
+  const OFF offf = (rowl * (2 * RW) + 2 * col) * 8;
   // lanes without a cell load the first column of the lane-independent row instead (in the
   // arrays or their guard rows)
-  const OFF sfw = (OFF)d.HL * (kCoefWords * kRow * 8), sfb = (OFF)d.HL * (kRow * 8 * NC),
-            sff = (OFF)d.HL * (2 * kRow * 8);
+  const OFF sfw = (OFF)d.HL * (kCoefWords * RW * 8), sfb = (OFF)d.HL * (RW * 8 * NC),
+            sff = (OFF)d.HL * (2 * RW * 8);
   struct Level {
     double w[kCoefWords], f0, f1;
     V b;
@@ -717,20 +729,21 @@ __global__ __launch_bounds__(512, 2) void k_gs_tiles(GsArgs a, Ops ops) {
   auto load = [&](int T, int r, Level& v) {
     const bool ok = col_ok[r] & ((unsigned)(T - lane - r) < (unsigned)X);
     const long row = slot_row(d, jt - 1, T - r - s, min(max(k0 + r, 0), d.Z - 1));
-    const char* const pw = at(W + row * (kCoefWords * kRow), ok ? offw : sfw);
+    const double* const pw = W + row * (kCoefWords * RW);
+    const OFF ow = ok ? offw : sfw;
 #pragma unroll
     for (int q = 0; q < kCoefWords; q += 2) {
-      const double2 x = *reinterpret_cast<const double2*>(pw + coef_word(q) * 8);
+      const double2 x = *reinterpret_cast<const double2*>(at(pw + coef_word(RW, q), ow));
       v.w[q] = x.x;
       v.w[q + 1] = x.y;
     }
     if constexpr (FALL) {
       const double2 x =
-          *reinterpret_cast<const double2*>(at(a.wf + row * (2 * kRow), ok ? offf : sff));
+          *reinterpret_cast<const double2*>(at(a.wf + row * (2 * RW), ok ? offf : sff));
       v.f0 = x.x;
       v.f1 = x.y;
     }
-    v.b = *reinterpret_cast<const V*>(at(B + row * (kRow * NC), ok ? offb : sfb));
+    v.b = *reinterpret_cast<const V*>(at(B + row * (RW * NC), ok ? offb : sfb));
     v.ok = ok;
   };
   Level lv[D][KR];
@@ -952,7 +965,7 @@ struct asam_tr_ctx {
   int order_kr = 0;
   std::vector<int> groups;  // sweeps per launch of a preconditioner application
   double *vx = nullptr, *vb = nullptr, *vr = nullptr, *vrt = nullptr, *vrh = nullptr;
-  double *vp = nullptr, *vph = nullptr, *vt = nullptr, *vv = nullptr, *vh = nullptr;
+  double *vp = nullptr, *vph = nullptr, *vt = nullptr, *vv = nullptr;
   double *partial = nullptr, *dots = nullptr;
   int *sync = nullptr;  // ticket, error word, set-up flag
   int sync_n = 0;
@@ -1003,9 +1016,10 @@ static void trfree(asam_tr_ctx* c, void* p) {
   (void)hipFree(p);
 }
 
-// A skewed array of `words` words per slot of n slots, with its guard rows.
+// A skewed array of `words` words per slot of n slots, with its guard rows (of up to two
+// components a slot).
 static int skew_alloc(asam_tr_ctx* c, double** p, long n, int words) {
-  const size_t guard = (size_t)kGuardRows * kRow * words * 2;
+  const size_t guard = (size_t)kGuardRows * c->d.RW * words * 2;
   int rc = tralloc(c, p, (size_t)n * words + 2 * guard);
   if (!rc) *p += guard;
   return rc;
@@ -1054,12 +1068,30 @@ extern "C" int asam_tr_create(asam_tr_ctx** out, const asam_tr_grid* g) {
   // the sweeps of an application in launches of nearly equal size
   const int total = g->iterg + 1, nl = (total + kMaxSweeps - 1) / kMaxSweeps;
   for (int q = 0; q < nl; ++q) c->groups.push_back(total / nl + (q < total % nl ? 1 : 0));
-  // y-tiles that cover Y columns at every sweep's shift
-  const int span = d.Y + c->groups[0] - 1;
-  d.NJ = (span + kMaxCols - 1) / kMaxCols;
-  d.TW = (span + d.NJ - 1) / d.NJ;
-  d.HL = d.X + d.TW - 1;
-  d.slots = (long)d.Z * d.NJ * d.HL * kRow;
+  // Components that the sweeps hold at most: groups of two repeat the first one where none is
+  // left of its operator kind, and are taken only if that makes fewer groups than components.
+  const long places = c->nc <= 2 ? c->nc : c->nc == 3 ? 4 : c->nc + 2 + c->nc % 2;
+  // y-tiles of at most `cols` columns that cover Y columns at every sweep's shift.  Rows of
+  // kRow entries, of the columns in use where these are few; `compact`: of the columns, rounded
+  // up to whole 128-byte lines where that adds at most a quarter.
+  auto set_tiles = [&](int cols, bool compact) {
+    const int span = d.Y + c->groups[0] - 1;
+    d.NJ = (span + cols - 1) / cols;
+    d.TW = (span + d.NJ - 1) / d.NJ;
+    d.ZW = d.NJ == 1 ? d.Y : d.TW;
+    d.HL = d.X + d.ZW - 1;
+    const int lines = (d.ZW + 7) / 8 * 8;
+    d.RW = d.ZW < 27 ? d.ZW : !compact ? kRow : 4 * lines <= 5 * d.ZW ? lines : d.ZW;
+    d.slots = (long)d.Z * d.NJ * d.HL * d.RW;
+  };
+  // Bytes of the skewed arrays, which must not keep a block off the card.  With few cells in x,
+  // wide tiles hold little but skew: above 4 GiB, tiles of X + Z columns (1x100000x20, four
+  // components: 14 GB instead of 35).  Above 32 GiB, compact rows (40000x48x100, one
+  // component: 42 GB instead of 84).
+  const long per = 8 * (2 * kCoefWords + 2 + 2 * places);
+  set_tiles(kMaxCols, false);
+  if (per * d.slots > (4L << 30) && d.X + d.Z < d.TW) set_tiles(d.X + d.Z, true);
+  else if (per * d.slots > (32L << 30)) set_tiles(kMaxCols, true);
   c->ops_mv.nc = c->ops_ps.nc = c->nc;
   for (int q = 0; q < kMaxComp; ++q) {
     c->ops_mv.op[q] = c->ops_ps.op[q] = ASAM_TR_POT;
@@ -1074,13 +1106,10 @@ extern "C" int asam_tr_create(asam_tr_ctx** out, const asam_tr_grid* g) {
   rc |= skew_alloc(c, &c->wmom, d.slots, kCoefWords);
   rc |= skew_alloc(c, &c->wpot, d.slots, kCoefWords);
   rc |= skew_alloc(c, &c->wf, d.slots, 2);
-  // groups of two: room for the places that they repeat, one per operator kind
-  const long places = c->nc == 1 ? 1 : c->nc + std::min(c->nc, 3);
   rc |= skew_alloc(c, &c->bs, places * d.slots, 1);
   rc |= skew_alloc(c, &c->xs, places * d.slots, 1);
   if (c->groups.size() > 1) rc |= skew_alloc(c, &c->ts, places * d.slots, 1);
-  double** vecs[] = {&c->vx, &c->vb, &c->vr, &c->vrt, &c->vrh, &c->vp, &c->vph, &c->vt, &c->vv,
-                     &c->vh};
+  double** vecs[] = {&c->vx, &c->vb, &c->vr, &c->vrt, &c->vrh, &c->vp, &c->vph, &c->vt, &c->vv};
   for (double** v : vecs) rc |= tralloc(c, v, V);
   rc |= tralloc(c, &c->partial, 2 * (size_t)std::max((long)blocks_for(d.m, 256), step_blocks(c)));
   rc |= tralloc(c, &c->dots, 2);
@@ -1233,11 +1262,14 @@ static void tiles_launch(asam_tr_ctx* c, const GsArgs& a, unsigned blocks) {
   const size_t lds = 2 * (size_t)a.M * (KR + 1) * kLdsRow * sizeof(double) * NC;
   const dim3 threads(64 * (a.M + 2));
   // 32-bit byte offsets within a tile's rows, except for blocks of about a million cells in x
-  if ((long)(a.d.HL + 1) * (kCoefWords * kRow * 8) < (1L << 32))
-    k_gs_tiles<NC, KR, D, FALL, DIV, unsigned><<<blocks, threads, lds, c->stream>>>(a,
-                                                                                       c->ops_ps);
+  if ((long)(a.d.HL + 1) * (kCoefWords * a.d.RW * 8) >= (1L << 32))
+    k_gs_tiles<NC, KR, D, FALL, DIV, 0, unsigned long>
+        <<<blocks, threads, lds, c->stream>>>(a, c->ops_ps);
+  else if (a.d.RW == kRow)
+    k_gs_tiles<NC, KR, D, FALL, DIV, kRow, unsigned>
+        <<<blocks, threads, lds, c->stream>>>(a, c->ops_ps);
   else
-    k_gs_tiles<NC, KR, D, FALL, DIV, unsigned long>
+    k_gs_tiles<NC, KR, D, FALL, DIV, 0, unsigned>
         <<<blocks, threads, lds, c->stream>>>(a, c->ops_ps);
 }
 
@@ -1333,7 +1365,8 @@ static long sweep_blocks(const asam_tr_ctx* c, int KR) {
   return (long)c->d.NJ * ((c->d.Z + c->groups[0] - 1 + KR - 1) / KR);
 }
 static long sweep_records(const asam_tr_ctx* c, int KR, int M) {
-  return sweep_blocks(c, KR) * (c->d.X + c->d.TW + KR - 2) * M * (c->d.TW + KR);
+  return sweep_blocks(c, KR) * (c->d.X + c->d.TW + KR - 2) * M *
+         (c->d.ZW + (c->d.NJ == 1 ? 0 : KR));
 }
 
 // Block order and boundary records of the default shape, for `places` components.
@@ -1547,8 +1580,8 @@ extern "C" int asam_tr_matvec(asam_tr_ctx* c, const double* x, double* y, int in
   if (!c || !x || !y) return trfail(c, ASAM_E_INVALID, "null argument");
   TRY(check_ready(c, c->ops_mv));
   TRCHK(c, hipSetDevice(c->device));
-  TRCHK(c, hipMemcpyAsync(c->vh, x, vbytes(c), hipMemcpyHostToDevice, c->stream));
-  TRY(launch_matvec(c, c->vh, c->vt, init));
+  TRCHK(c, hipMemcpyAsync(c->vx, x, vbytes(c), hipMemcpyHostToDevice, c->stream));
+  TRY(launch_matvec(c, c->vx, c->vt, init));
   TRCHK(c, hipMemcpyAsync(y, c->vt, vbytes(c), hipMemcpyDeviceToHost, c->stream));
   TRCHK(c, hipStreamSynchronize(c->stream));
   return 0;
@@ -1558,8 +1591,8 @@ extern "C" int asam_tr_psolve(asam_tr_ctx* c, const double* x, double* y) {
   if (!c || !x || !y) return trfail(c, ASAM_E_INVALID, "null argument");
   TRY(check_ready(c, c->ops_ps));
   TRCHK(c, hipSetDevice(c->device));
-  TRCHK(c, hipMemcpyAsync(c->vh, x, vbytes(c), hipMemcpyHostToDevice, c->stream));
-  TRY(launch_psolve(c, c->vh, c->vt));
+  TRCHK(c, hipMemcpyAsync(c->vx, x, vbytes(c), hipMemcpyHostToDevice, c->stream));
+  TRY(launch_psolve(c, c->vx, c->vt));
   TRCHK(c, hipMemcpyAsync(y, c->vt, vbytes(c), hipMemcpyDeviceToHost, c->stream));
   TRCHK(c, hipStreamSynchronize(c->stream));
   return check_gs_error(c);
