@@ -155,23 +155,28 @@ __global__ __launch_bounds__(256) void k_matvec(Dims d, const double* __restrict
 // ------------------------------------------------------------------ division
 // t / dg from y = 1/dg (correctly rounded): two residual corrections of t*y.  The first leaves
 // a quotient within an ulp and the second rounds correctly (Markstein, IBM J. Res. Dev. 34,
-// 1990), as long as no residual underflows: |t| above 2^-960 and |dg| within 2^+-500 (the
-// set-up notes a matrix with another diagonal, and the sweeps then divide).  Five dependent
-// operations in the sweep's serial chain instead of the division's dozen.  The caller divides
-// where the result is NaN, infinite or subnormal (gs_odd).  The sign is that of t*y, also for
-// a zero.
+// 1990), as long as no residual underflows, which |t| of 2^-960 and more ensures: |dg| of 2^-60
+// and more (to 2^500; the set-up notes a matrix with another diagonal, and the sweeps then
+// divide) and quotients of 2^-900 and more.  Five dependent operations in the sweep's serial
+// chain instead of the division's dozen.  The sign is that of t*y, also for a zero.
 __device__ __forceinline__ double gs_divide(double t, double dg, double y) {
   const double q0 = t * y;
   const double q1 = __builtin_fma(__builtin_fma(-q0, dg, t), y, q0);
   const double q2 = __builtin_fma(__builtin_fma(-q1, dg, t), y, q1);
   return __builtin_copysign(q2, q0);
 }
-__device__ __forceinline__ bool gs_odd(double q) {
-  return __builtin_amdgcn_class(q, 0x003 | 0x204 | 0x090);  // NaN, infinite, subnormal
+// The caller divides where the quotient of a t other than zero is below 2^-900, infinite or NaN:
+// where this is at least kOddKey (the high word without its sign, from 2^-900 on; smaller ones
+// wrap).  A maximum of such keys takes vector instructions only: as comparisons joined in scalar
+// registers the test cost 2% of the launch at 256x256x64, this way 0.5%.
+constexpr unsigned kOddLow = 2 * (1023u - 900u) << 20, kOddKey = (2 * 2047u << 20) - kOddLow;
+__device__ __forceinline__ unsigned gs_key(double t, double q) {
+  const unsigned u = ((unsigned)__double2hiint(q) << 1) - kOddLow;
+  return t != 0.0 ? u : 0u;
 }
 __device__ __forceinline__ bool gs_plain_diag(double dg) {
   const double m = fabs(dg);
-  return m >= 0x1p-500 && m <= 0x1p500;
+  return m >= 0x1p-60 && m <= 0x1p500;
 }
 
 // ------------------------------------------------------------------ skewed layout
@@ -767,7 +772,7 @@ __global__ __launch_bounds__(512, 2) void k_gs_tiles(GsArgs a, Ops ops) {
         Level(&v)[KR] = lv[u % D];
         // the chains of all levels and components side by side, without a branch
         double t[KR][NC], x[KR][NC];
-        bool odd = false;
+        unsigned most = 0;
 #pragma unroll
         for (int r = 0; r < KR; ++r) {
           V o0, o1, o2;
@@ -794,6 +799,7 @@ __global__ __launch_bounds__(512, 2) void k_gs_tiles(GsArgs a, Ops ops) {
         }
 #pragma unroll
         for (int r = 0; r < KR; ++r) {
+          unsigned key = 0;
 #pragma unroll
           for (int c = 0; c < NC; ++c) {
             if constexpr (DIV) {
@@ -802,11 +808,12 @@ __global__ __launch_bounds__(512, 2) void k_gs_tiles(GsArgs a, Ops ops) {
               x[r][c] = t[r][c] / dg;
             } else {
               x[r][c] = gs_divide(t[r][c], v[r].w[6], v[r].w[7]);
-              odd |= gs_odd(x[r][c]) & v[r].ok;
+              key = max(key, gs_key(t[r][c], x[r][c]));
             }
           }
+          most = max(most, v[r].ok ? key : 0u);
         }
-        if (!DIV && __builtin_expect(__ballot(odd) != 0, 0)) {
+        if (!DIV && __builtin_expect(__ballot(most >= kOddKey) != 0, 0)) {
 #pragma unroll
           for (int r = 0; r < KR; ++r)
 #pragma unroll
