@@ -928,9 +928,11 @@ __global__ __launch_bounds__(256) void k_step_full(Dims d, int nc, double alpha,
   block_reduce_store<2>(acc, partial, blockIdx.x, threadIdx.x, 256, gridDim.x);
 }
 // Fixed-order sums of the two partial sums of nblk blocks: thread t adds partials t, t + 1024,
-// ..., then the block tree; every run gives the same bits.
+// ..., then the block tree; every run gives the same bits.  out[2]: the sweeps' error word.
 __global__ __launch_bounds__(1024) void k_dot_fin(const double* __restrict__ partial, int nblk,
+                                                  const int* __restrict__ err,
                                                   double* __restrict__ out) {
+  if (threadIdx.x == 0) out[2] = *err;
   double v[2] = {0.0, 0.0};
 #pragma unroll 4
   for (int b = threadIdx.x; b < nblk; b += 1024) {
@@ -1119,11 +1121,11 @@ extern "C" int asam_tr_create(asam_tr_ctx** out, const asam_tr_grid* g) {
   double** vecs[] = {&c->vx, &c->vb, &c->vr, &c->vrt, &c->vrh, &c->vp, &c->vph, &c->vt, &c->vv};
   for (double** v : vecs) rc |= tralloc(c, v, V);
   rc |= tralloc(c, &c->partial, 2 * (size_t)std::max((long)blocks_for(d.m, 256), step_blocks(c)));
-  rc |= tralloc(c, &c->dots, 2);
+  rc |= tralloc(c, &c->dots, 3);
   c->sync_n = 3;  // ticket, error word, set-up flag
   rc |= tralloc(c, &c->sync, (size_t)c->sync_n);
   if (rc) return bail(ASAM_E_NOMEM);
-  if (hipHostMalloc((void**)&c->host_dots, 2 * sizeof(double), hipHostMallocDefault) != hipSuccess)
+  if (hipHostMalloc((void**)&c->host_dots, 3 * sizeof(double), hipHostMallocDefault) != hipSuccess)
     return bail(ASAM_E_NOMEM);
   if (hipMemsetAsync(c->sync, 0, sizeof(int) * c->sync_n, c->stream) != hipSuccess ||
       hipStreamSynchronize(c->stream) != hipSuccess)
@@ -1425,7 +1427,6 @@ static int psolve_nc(asam_tr_ctx* c, const double* x, double* y) {
   const Dims& d = c->d;
   const Groups gr = make_groups(c, NC);
   const int levels = d.Z * gr.n;
-  k_zero_int<<<1, 64, 0, c->stream>>>(c->sync + 1, 1);
   k_skew_vec<NC><<<dim3(d.NJ * ((d.HL + kVecH - 1) / kVecH), 1, levels), 256, 0, c->stream>>>(
       d, gr, x, c->bs);
   TRCHK(c, hipGetLastError());
@@ -1442,22 +1443,31 @@ static int launch_psolve(asam_tr_ctx* c, const double* x, double* y) {
   return sweep_shape(c).NC == 2 ? psolve_nc<2>(c, x, y) : psolve_nc<1>(c, x, y);
 }
 
+// The error word of the sweeps' waits: cleared when a call begins, read before it returns.
+static const char kWaited[] = "Gauss-Seidel sweep: a workgroup waited past its limit";
+static int clear_gs_error(asam_tr_ctx* c) {
+  k_zero_int<<<1, 64, 0, c->stream>>>(c->sync + 1, 1);
+  TRCHK(c, hipGetLastError());
+  return 0;
+}
 static int check_gs_error(asam_tr_ctx* c) {
   int e = 0;
   TRCHK(c, hipMemcpyAsync(&e, c->sync + 1, sizeof(int), hipMemcpyDeviceToHost,
                           c->stream));
   TRCHK(c, hipStreamSynchronize(c->stream));
-  if (e) return trfail(c, ASAM_E_HIP, "Gauss-Seidel sweep: a workgroup waited past its limit");
+  if (e) return trfail(c, ASAM_E_HIP, kWaited);
   return 0;
 }
 
-// The two sums of the nblk blocks launched last; results on the host.
+// The two sums of the nblk blocks launched last; results on the host.  Fails where a sweep
+// before them gave up waiting.
 static int sums(asam_tr_ctx* c, long nblk, double* out) {
-  k_dot_fin<<<1, 1024, 0, c->stream>>>(c->partial, (int)nblk, c->dots);
+  k_dot_fin<<<1, 1024, 0, c->stream>>>(c->partial, (int)nblk, c->sync + 1, c->dots);
   TRCHK(c, hipGetLastError());
-  TRCHK(c, hipMemcpyAsync(c->host_dots, c->dots, 2 * sizeof(double), hipMemcpyDeviceToHost,
+  TRCHK(c, hipMemcpyAsync(c->host_dots, c->dots, 3 * sizeof(double), hipMemcpyDeviceToHost,
                           c->stream));
   TRCHK(c, hipStreamSynchronize(c->stream));
+  if (c->host_dots[2] != 0.0) return trfail(c, ASAM_E_HIP, kWaited);
   out[0] = c->host_dots[0];
   out[1] = c->host_dots[1];
   return 0;
@@ -1483,6 +1493,7 @@ static int solve_dev(asam_tr_ctx* c, double* x, const double* b, int* maxiter, d
          *v = c->vv;
   const int MaxIter = *maxiter;
   const double Tol = *tol;
+  TRY(clear_gs_error(c));
   TRY(launch_matvec(c, x, r, 1));  // MatVecChem(r, A, x)
   inf.matvecs = 1;
   const Dims& d = c->d;
@@ -1548,7 +1559,7 @@ static int solve_dev(asam_tr_ctx* c, double* x, const double* b, int* maxiter, d
   }
   inf.rnorm = (inf.status == ASAM_BREAKDOWN) ? rnorm : *tol;
   if (!std::isfinite(rnorm)) return trfail(c, ASAM_E_NAN, "non-finite residual");
-  TRY(check_gs_error(c));
+  TRCHK(c, hipStreamSynchronize(c->stream));  // the last update of x
   if (info) *info = inf;
   return 0;
 }
@@ -1566,6 +1577,7 @@ extern "C" int asam_tr_psolve_device(asam_tr_ctx* c, const double* x, double* y)
   if (!c || !x || !y) return trfail(c, ASAM_E_INVALID, "null argument");
   TRY(check_ready(c, c->ops_ps));
   TRCHK(c, hipSetDevice(c->device));
+  TRY(clear_gs_error(c));
   TRY(launch_psolve(c, x, y));
   return check_gs_error(c);
 }
@@ -1599,6 +1611,7 @@ extern "C" int asam_tr_psolve(asam_tr_ctx* c, const double* x, double* y) {
   TRY(check_ready(c, c->ops_ps));
   TRCHK(c, hipSetDevice(c->device));
   TRCHK(c, hipMemcpyAsync(c->vx, x, vbytes(c), hipMemcpyHostToDevice, c->stream));
+  TRY(clear_gs_error(c));
   TRY(launch_psolve(c, c->vx, c->vt));
   TRCHK(c, hipMemcpyAsync(y, c->vt, vbytes(c), hipMemcpyDeviceToHost, c->stream));
   TRCHK(c, hipStreamSynchronize(c->stream));
@@ -1645,6 +1658,7 @@ extern "C" int asam_tr_time_kernel(asam_tr_ctx* c, int which, int reps, double* 
   if (!c || !ms || reps < 1 || which < 0 || which > 2) return trfail(c, ASAM_E_INVALID, "argument");
   TRY(check_ready(c, which == 1 ? c->ops_mv : c->ops_ps));
   TRCHK(c, hipSetDevice(c->device));
+  TRY(clear_gs_error(c));
   hipEvent_t e0, e1;
   TRCHK(c, hipEventCreate(&e0));
   TRCHK(c, hipEventCreate(&e1));
