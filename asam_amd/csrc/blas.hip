@@ -174,13 +174,14 @@ void launch_gm_dot(hipStream_t s, long n, int vt, const void* w, const void* v0,
 //
 // hsrc: null, or the partial sums of the pass before (NP products, then the g_ab); each
 // workgroup adds them up in the same order and the first one records the h_a in H.  The first
-// pass of a step has NP = 1 and takes h_0 from H.
+// pass of a step has NP = 1 and takes h_0 from H.  The vectors are allocations of their own, so
+// 16-byte packs of them are aligned.
 constexpr int kMgsSums = kMgsBlock + kMgsBlock * (kMgsBlock - 1) / 2;
 struct MgsVecs {
   const void* prev[kMgsBlock];
   const void* next[kMgsBlock];
 };
-template <typename VT, bool PK, int NP, int NN>
+template <typename VT, int NP, int NN>
 __global__ __launch_bounds__(256) void k_mgs(long n, VT* __restrict__ w, MgsVecs vs, int k0,
                                              int i, KState* st, double* partial,
                                              const double* hsrc) {
@@ -248,7 +249,7 @@ __global__ __launch_bounds__(256) void k_mgs(long n, VT* __restrict__ w, MgsVecs
   };
   const long stride = (long)gridDim.x * blockDim.x;
   const long gid = blockIdx.x * (long)blockDim.x + tid;
-  constexpr int W = PK ? Pk<VT>::W : 1;
+  constexpr int W = Pk<VT>::W;
   const long nc = n / W;
   // U turns of the grid-stride loop at a time, all loads first
   constexpr int U = NP + NN >= 5 ? 1 : NP + NN >= 3 ? 2 : 4;
@@ -259,20 +260,11 @@ __global__ __launch_bounds__(256) void k_mgs(long n, VT* __restrict__ w, MgsVecs
     for (int u = 0; u < U; ++u) {
       const long c = c0 + u * stride;
       if (CHK && c >= nc) break;
-      auto ld = [&](const VT* v) {
-        if constexpr (PK) {
-          return ldpk(v, c);
-        } else {
-          Pk<VT> r;
-          r.v[0] = v[c];
-          return r;
-        }
-      };
-      wl[u] = ld(w);
+      wl[u] = ldpk(w, c);
 #pragma unroll
-      for (int a = 0; a < NP; ++a) pl[u][a] = ld((const VT*)vs.prev[a]);
+      for (int a = 0; a < NP; ++a) pl[u][a] = ldpk((const VT*)vs.prev[a], c);
 #pragma unroll
-      for (int a = 0; a < NN; ++a) xl[u][a] = ld((const VT*)vs.next[a]);
+      for (int a = 0; a < NN; ++a) xl[u][a] = ldpk((const VT*)vs.next[a], c);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -287,37 +279,33 @@ __global__ __launch_bounds__(256) void k_mgs(long n, VT* __restrict__ w, MgsVecs
         for (int a = 0; a < NN; ++a) x[a] = xl[u][a].v[j];
         wl[u].v[j] = elem(wl[u].v[j], p, x);
       }
-      if constexpr (PK) stpk(w, c, wl[u]);
-      else w[c] = wl[u].v[0];
+      stpk(w, c, wl[u]);
     }
   };
   long c = gid;
   for (; c + (U - 1) * stride < nc; c += U * stride) turns(c, std::false_type{});
   if (c < nc) turns(c, std::true_type{});
-  if constexpr (PK) {  // the n mod W last elements
-    const long e = nc * W + gid;
-    if (e < n) {
-      VT p[NP], x[NN + 1];
+  const long e = nc * W + gid;  // the n mod W last elements
+  if (e < n) {
+    VT p[NP], x[NN + 1];
 #pragma unroll
-      for (int a = 0; a < NP; ++a) p[a] = ((const VT*)vs.prev[a])[e];
+    for (int a = 0; a < NP; ++a) p[a] = ((const VT*)vs.prev[a])[e];
 #pragma unroll
-      for (int a = 0; a < NN; ++a) x[a] = ((const VT*)vs.next[a])[e];
-      w[e] = elem(w[e], p, x);
-    }
+    for (int a = 0; a < NN; ++a) x[a] = ((const VT*)vs.next[a])[e];
+    w[e] = elem(w[e], p, x);
   }
   block_reduce_store<NO>(acc, partial, blockIdx.x, tid, 256, kMgsStride);
 }
 
 int mgs_blocks(long n) { return std::min(blas_blocks(n), 512); }
 
-template <typename VT, bool PK>
+template <typename VT>
 static void mgs_go(hipStream_t s, long n, VT* w, const MgsVecs& v, int np, int nn, int k0, int i,
                    KState* st, double* partial, const double* hsrc) {
   const dim3 grid(mgs_blocks(n)), wg(256);
 #define MGS(P, N)                                                                            \
   if (np == P && nn == N) {                                                                  \
-    hipLaunchKernelGGL((k_mgs<VT, PK, P, N>), grid, wg, 0, s, n, w, v, k0, i, st, partial,   \
-                       hsrc);                                                                \
+    hipLaunchKernelGGL((k_mgs<VT, P, N>), grid, wg, 0, s, n, w, v, k0, i, st, partial, hsrc); \
     return;                                                                                  \
   }
   // a block that is not full is the last one
@@ -330,16 +318,10 @@ void launch_mgs(hipStream_t s, long n, int vt, void* const* vs, int k0, int np, 
   static_assert(kMgsBlock == 3, "the combinations of mgs_go");
   void* const w = vs[i + 1];
   MgsVecs v{};
-  bool pk = al16(w);
-  for (int a = 0; a < np; ++a) pk = al16(v.prev[a] = vs[k0 + a]) && pk;
-  for (int a = 0; a < nn; ++a) pk = al16(v.next[a] = vs[k0 + np + a]) && pk;
-  if (vt == 0) {
-    if (pk) mgs_go<double, true>(s, n, (double*)w, v, np, nn, k0, i, st, partial, hsrc);
-    else mgs_go<double, false>(s, n, (double*)w, v, np, nn, k0, i, st, partial, hsrc);
-  } else {
-    if (pk) mgs_go<float, true>(s, n, (float*)w, v, np, nn, k0, i, st, partial, hsrc);
-    else mgs_go<float, false>(s, n, (float*)w, v, np, nn, k0, i, st, partial, hsrc);
-  }
+  for (int a = 0; a < np; ++a) v.prev[a] = vs[k0 + a];
+  for (int a = 0; a < nn; ++a) v.next[a] = vs[k0 + np + a];
+  if (vt == 0) mgs_go<double>(s, n, (double*)w, v, np, nn, k0, i, st, partial, hsrc);
+  else mgs_go<float>(s, n, (float*)w, v, np, nn, k0, i, st, partial, hsrc);
 }
 
 struct ZList {
