@@ -522,14 +522,31 @@ def projection_leg(s, p, steps, tol):
                        "GBs": round(ub / (ms_u * 1e-3) / 1e9, 1)}}
 
 
+def gs_launch(nx, ny, nz, ncomp, iterg, ms_per_sweep):
+    """The largest launch of Gauss-Seidel sweeps of a preconditioner application (the 1 + iterg
+    sweeps go in launches of nearly equal size, six at most), from the time per sweep that
+    time_kernel(0) gives, the reset of the boundary records included.  Its algorithmic bytes
+    are the 7 coefficients once and b and the result once per component: old values stay on
+    the chip and later sweeps take the coefficients from the caches."""
+    total = 1 + iterg
+    sweeps = -(-total // -(-total // 6))
+    x, y, z = nx + 2, ny + 2, nz + 2
+    bytes_ = x * y * z * (7 + 2 * ncomp) * 8
+    ms = ms_per_sweep * sweeps
+    gbs = bytes_ / (ms * 1e-3) / 1e9
+    return {"avg_launch_us": round(ms * 1e3, 1), "sweeps": sweeps, "bytes": bytes_,
+            "GBs": round(gbs, 1), "frac": round(gbs / HBM_PEAK_GBS, 4),
+            "bound": f"latency: {sweeps} sweeps, two hyperplanes apart, are a chain of "
+                     f"{x + y + z + 2 * sweeps} steps"}
+
+
 def transport_leg(steps, with_cpu, cpu_seconds=15.0, ncomp=4, tol=1e-6, maxiter=30):
     """The transport stage solve (BiCGStabChemSp, reference MODULE/SpMatrix4CellPar_Mod.f90
     :140-243) of `ncomp` tracers on the 256x256x64 cut-cell grid: upwind advection and
     diffusion Jacobian from the stage velocities, a per-cell chemistry LU, x0 = 0 and the
     reference's BiCGStabTol / BiCGStabMaxIter defaults (Control_Mod.f90:580-581).  Solves
-    on resident device vectors; the Gauss-Seidel sweep's algorithmic bytes per launch are
-    ncomp * m * (7 coefficients + b + old x + new x) words; the oracle solve is timed on
-    the host cores beside it."""
+    on resident device vectors; the launch of the Gauss-Seidel sweeps as in gs_launch; the
+    oracle solve is timed on the host cores beside it."""
     from asam_amd import transport, workload
     p = workload.config(2, np1=1)
     tp = workload.transport_problem(p, ncomp=ncomp)
@@ -548,7 +565,6 @@ def transport_leg(steps, with_cpu, cpu_seconds=15.0, ncomp=4, tol=1e-6, maxiter=
     ms_sweep = s.time_kernel(0, 10)
     ms_mv = s.time_kernel(1, 10)
     ms_ps = s.time_kernel(2, 3)
-    sweep_bytes = tp.ncomp * tp.m * 10 * 8
     mv_bytes = tp.m * (7 + 3 * tp.ncomp + (tp.ncomp ** 2 if tp.lu is not None else 0)) * 8
     med = float(np.median(times))
     out = {"workload": f"256x256x64 cut-cell transport stage solve, {ncomp} tracers "
@@ -557,11 +573,7 @@ def transport_leg(steps, with_cpu, cpu_seconds=15.0, ncomp=4, tol=1e-6, maxiter=
            "solves_per_s": round(1.0 / med, 3), "ms_per_solve": round(1e3 * med, 3),
            "maxiter_out": infos[-1][0], "tol_out": infos[-1][1], "info": infos[-1][2],
            "tuning": s.get_tuning().as_dict(),
-           "gs_sweep": {"avg_launch_us": round(ms_sweep * 1e3, 1), "bytes": sweep_bytes,
-                        "GBs": round(sweep_bytes / (ms_sweep * 1e-3) / 1e9, 1),
-                        "frac": round(sweep_bytes / (ms_sweep * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
-                        "bound": "latency: one lexicographic sweep is a chain of "
-                                 f"{(tp.nx + 2) + (tp.ny + 2) + (tp.nz + 2) - 2} hyperplanes"},
+           "gs_sweeps": gs_launch(tp.nx, tp.ny, tp.nz, tp.ncomp, tp.iterg, ms_sweep),
            "matvec": {"avg_launch_us": round(ms_mv * 1e3, 1), "bytes": mv_bytes,
                       "GBs": round(mv_bytes / (ms_mv * 1e-3) / 1e9, 1)},
            "psolve_ms": round(ms_ps, 3)}

@@ -78,7 +78,8 @@ typedef struct {
   int reserved;
 } asam_tr_tuning;
 
-/* Creates the context and its device workspace (no per-call allocation). */
+/* Creates the context and its device workspace (no per-call allocation; a gs_rows that cuts
+ * the block finer grows the boundary records at the next application). */
 int asam_tr_create(asam_tr_ctx **ctx, const asam_tr_grid *grid);
 int asam_tr_destroy(asam_tr_ctx *ctx);
 const char *asam_tr_last_error(const asam_tr_ctx *ctx);
@@ -121,8 +122,8 @@ int asam_tr_solve_device(asam_tr_ctx *ctx, double *x, const double *b, int *maxi
 int asam_tr_get_tuning(const asam_tr_ctx *ctx, asam_tr_tuning *t);
 int asam_tr_set_tuning(asam_tr_ctx *ctx, const asam_tr_tuning *t);
 /* Device time of the kernels on the context's own buffers, averaged over reps launches
- * (HIP events on the context's stream): which 0 = one Gauss-Seidel sweep over all
- * components, 1 = the operator (MatVec), 2 = one whole PSolve.  No counterpart in the
+ * (HIP events on the context's stream): which 0 = a launch of Gauss-Seidel sweeps over all
+ * components, divided by its number of sweeps, 1 = the operator (MatVec), 2 = one whole PSolve.  No counterpart in the
  * reference (measurement). */
 int asam_tr_time_kernel(asam_tr_ctx *ctx, int which, int reps, double *ms);
 
