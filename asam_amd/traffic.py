@@ -36,7 +36,7 @@ def kernel_class(name: str):
         kind = "apply" if m.group(1).startswith("apply") else "line"
         # the first floating type in the template list is the coefficient type
         return f"{kind}_{'fp64' if m.group(2) == 'double' else 'fp32'}"
-    m = re.search(r"k_(bicg_update|mgs|gmres_update|cgs_dots|cgs_update)<(double|float)[,>]",
+    m = re.search(r"k_(bicg_update|gm_dot|mgs|gmres_update|cgs_dots|cgs_update)<(double|float)[,>]",
                   name)
     if m:
         return f"blas_{'fp64' if m.group(2) == 'double' else 'fp32'}"
