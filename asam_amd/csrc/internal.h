@@ -96,16 +96,19 @@ __host__ __device__ inline long fac_index(const Geom& g, int i, int j, int k) {
 //   tiles            64        192       291       480         600         1024
 //   2x2 FP64      466/427   600/565   711/690   2112/2124   2696/2790   5222/5231
 //   1-comp. FP64  318/293   434/405   491/471   1114/1119   1350/1337   2603/2657
+// Up to 291 tiles both ends win by 3 to 8%; at 480 the two are equal to half a percent; at 600
+// 2x2 blocks lose 3% and one component wins 1%, which it loses again at 1024.  So the line may
+// lie anywhere from 291 to 600, and one line serves both.
 // The FP32 factors of a mixed solve always go from the bottom up (there 64 tiles of 2x2 blocks
 // would take 389 us for 436): the other order rounds every entry differently, and that moves a
 // solution refined to 1e-8 by up to 2.4e-9 of its norm (128x128x64).
 constexpr int line_halves(long tiles) { return tiles <= 512 ? 2 : 1; }
 // Words per cell of the line solve's blocks towards the previous level of the elimination:
-// L_k, and with elimination from both ends U_k from the middle nz/2 up.  A 2x2 block couples two levels through one
-// face and is rank one, so it is stored as three words: L_k = (tz, 1)^T (-kz DUT, gz V) with
-// the face below and the cell below, U_k = (tz, 1)^T (-kz DUT, -gz V) with the face above and
-// the cell above.  With both ends L of the middle level lies in the bottom level's place,
-// which has no use of its own.
+// L_k, and with elimination from both ends U_k from the middle nz/2 up.  A 2x2 block couples
+// two levels through one face and is rank one, so it is stored as three words:
+// L_k = (tz, 1)^T (-kz DUT, gz V) with the face below and the cell below,
+// U_k = (tz, 1)^T (-kz DUT, -gz V) with the face above and the cell above.  With both ends L of
+// the middle level lies in the bottom level's place, which has no use of its own.
 constexpr int lower_words(int np1) { return np1 == 2 ? 3 : 1; }
 // Entries per line-factor array (tiled layout pads x to a multiple of 64).
 inline long fac_cells(const Geom& g) { return ((long)(g.nx + 63) / 64) * 64 * g.ny * g.nz; }

@@ -74,7 +74,7 @@ __device__ __forceinline__ V2<T> mtv(const M4<T>& q, V2<T> v) {  // q^T * v
 // wavefront takes levels 0..m-1 upwards, the second nz-1..m+1 downwards and then m, where the
 // halves meet; the back-substitution runs outwards from there.  That halves the serial chain
 // of a column and doubles the loads in flight, which counts where the grid has too few tiles
-// to hide either (see line_two_ended for both sides measured).  Kernel times, one / two:
+// to hide either (see line_halves for both sides measured).  Kernel times, one / two:
 // FP64 64x64x40 one component 12.4 / 9.1 us, 2x2 17.8 / 12.9 us; transposed 2x2 130x97x40
 // 31 / 28 us.
 //

@@ -181,7 +181,7 @@ __device__ __forceinline__ bool gs_plain_diag(double dg) {
 
 // ------------------------------------------------------------------ skewed layout
 // Slot of cell (i, j, k) within an array of one word per cell: y-tile jt = j / TW, column
-// jj = j - jt*TW, row h = i + jj of the tile's HL = X + TW - 1 rows.
+// jj = j - jt*TW, row h = i + jj of the tile's HL rows (X + TW - 1; X + Y - 1 for one tile).
 constexpr int kCoefWords = 8;  // words per cell of a skewed matrix: see k_skew_coef
 constexpr int kMaxCols = 53;   // columns of a y-tile at most, see kMaxSweeps below
 // Entries of a row of the skewed layout for tiles of 27 columns and more.  Rows of 56 (the most
@@ -481,12 +481,12 @@ __device__ __forceinline__ bool is_sentinel(double v) {
 //  - Blocks are taken from an atomic ticket in an order in which a block's predecessors come
 //    first, so a block waits only for blocks that started before it; every wait is bounded.
 //
-// What bounds it: the dependent steps (about 2.1 us each at 256x256x64 with four components: as
-// much for the coefficient loads, 28 cycles of the L1 per 16-byte load of a wavefront, as for
-// the arithmetic, and what the blocks wait for each other's slowest step), and one hand-over of
-// 2.6 us per level block.  256x256x64, four components, 6 sweeps: 1.24 ms; one launch per sweep
-// with a pass for b - U x_old before it, rows handed over along y, took 4.3 ms.  101x77x50,
-// three components: 0.25 ms against 2.1 ms.
+// What bounds it: the chain of X + Y + Z + 2M steps.  256x256x64, four components, 6 sweeps:
+// 1.16 ms for 594 steps, 1.96 us each with the hand-overs between blocks counted in; the
+// coefficient loads (28 cycles of the L1 per 16-byte load of a wavefront) take as much of a step
+// as the arithmetic, and a block waits for the slowest step of those before it.  One launch per
+// sweep with a pass for b - U x_old before it, rows handed over along y, took 4.3 ms.
+// 101x77x50, three components: 0.24 ms against 2.1 ms.
 //
 // Term order of a row as in the reference (GaussSeidel_SpDiag :216-234): b, -U (+1, +X, +XY,
 // then JacFall's +XY), -L (-XY, -X, -1), / diag; products and sums are not contracted.  A

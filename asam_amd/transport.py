@@ -253,7 +253,8 @@ class TransportSolver:
         self._check(load().asam_tr_test_hold_boundary(self.h, int(bool(hold))))
 
     def time_kernel(self, which, reps=10):
-        """Device ms of one Gauss-Seidel sweep (0), one MatVec (1), one PSolve (2)."""
+        """Device ms of a launch of Gauss-Seidel sweeps per sweep (0), one MatVec (1), one
+        PSolve (2)."""
         ms = C.c_double()
         self._check(load().asam_tr_time_kernel(self.h, which, reps, C.byref(ms)))
         return ms.value

@@ -72,7 +72,7 @@ typedef struct {
 /* Launch shapes of the Gauss-Seidel sweeps (results do not depend on them). */
 typedef struct {
   int gs_rows;       /* z-levels per workgroup: 1, 2 or 3; 4..8 (default 8): by size */
-  int gs_chunk;      /* 2 or 4; has no effect */
+  int gs_chunk;      /* reserved: 2 or 4, without effect */
   int gs_spin_limit; /* polls of a boundary value before a block stops waiting for it (the
                         call then returns ASAM_E_HIP); 0: 4194304 */
   int reserved;
@@ -123,13 +123,13 @@ int asam_tr_get_tuning(const asam_tr_ctx *ctx, asam_tr_tuning *t);
 int asam_tr_set_tuning(asam_tr_ctx *ctx, const asam_tr_tuning *t);
 /* Device time of the kernels on the context's own buffers, averaged over reps launches
  * (HIP events on the context's stream): which 0 = a launch of Gauss-Seidel sweeps over all
- * components, divided by its number of sweeps, 1 = the operator (MatVec), 2 = one whole PSolve.  No counterpart in the
- * reference (measurement). */
+ * components, divided by its number of sweeps, 1 = the operator (MatVec), 2 = one whole
+ * PSolve.  No counterpart in the reference (measurement). */
 int asam_tr_time_kernel(asam_tr_ctx *ctx, int which, int reps, double *ms);
 
-/* Test hook, no counterpart in the reference: with hold != 0 no block publishes its last
- * row, so every later block waits for its boundary values until gs_spin_limit polls and
- * the sweep returns ASAM_E_HIP, every kernel still finishing normally.  For tests of the
+/* Test hook, no counterpart in the reference: with hold != 0 no block publishes its
+ * boundary, so every later block waits for its values until gs_spin_limit polls and
+ * the call returns ASAM_E_HIP, every kernel still finishing normally.  For tests of the
  * bounded wait (with a small gs_spin_limit); hold = 0 restores normal sweeps. */
 int asam_tr_test_hold_boundary(asam_tr_ctx *ctx, int hold);
 
