@@ -461,10 +461,10 @@ static int build_tables(asam_ens_ctx* c) {
   // multiples of a wide tile) by a common number of planes kp: the compute unit with most tiles
   // ends the launch, n tiles of kp planes take n (kp + 1) plane times, and below `busy` tiles a
   // unit idles.  (The rule for one domain counts kp + 2 and the wavefronts that have columns,
-  // which decide between its widths and small grids; here the width is given.)  Against whole columns of 256 by 2 tiles,
-  // solves of all members, us before / after: 7 members of 61 to 89 squared, 2x2, 3030/2253;
-  // 4 of 56 to 121, one component, 2274/1256; 7 of 51 to 159, 2x2, 4151/2982; 8 of 64 to
-  // 256, 2x2, 9379/8991.
+  // which decide between its widths and small grids; here the width is given.)  Against whole
+  // columns of 256 by 2 tiles, solves of all members, us before / after: 7 members of 61 to 89
+  // squared, 2x2, 3030/2253; 4 of 56 to 121, one component, 2274/1256; 7 of 51 to 159, 2x2,
+  // 4151/2982; 8 of 64 to 256, 2x2, 9379/8991.
   const bool balance =
       c->tune.apply_bx == 256 && c->tune.apply_zsplit == 1 && c->tune.apply_rows == 2;
   const int bx = c->abx = balance ? 64 : c->tune.apply_bx;
